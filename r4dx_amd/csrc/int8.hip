@@ -120,125 +120,103 @@ struct XqOut {
   signed char* a8[kXqMaxOut];
   float* sa[kXqMaxOut];
 };
-// the transformed block of (row, k0) for output o: lane l gets the f16 bits of elements l and l + 64
-// (s0, s1: suh of elements l and l + 64)
-__device__ __forceinline__ void xq_transform_s(float x0, float x1, float s0, float s1, int lane, float scale,
-                                               unsigned short& h0, unsigned short& h1) {
-  float v0 = x0 * s0;
-  float v1 = x1 * s1;
-  r4_fwht128_wave(v0, v1, lane);
-  h0 = r4_f16_rn(v0 * scale);
-  h1 = r4_f16_rn(v1 * scale);
+// Both kernels give a (row, 128-block) to 16 lanes, 8 adjacent elements per lane: the Hadamard stays in registers and DPP
+// moves (r4_fwht128_rows), a block's amax is a 16-lane DPP reduction, the loads are 16 bytes wide, and the lane that
+// transformed a value quantizes it. Two elements per lane went through the LDS crossbar for two Hadamard stages, the amax
+// and the quantizer's lane map (256 rows, before -> now: per-128 x 2 outputs at K 5120 9.0 -> 5.5 us; rows, silu at
+// K 17408 16.1 -> 13.6 us).
+// the f16 bits of the transformed 8 elements of this lane
+__device__ __forceinline__ void xq_transform8(const float (&x)[8], const float (&s)[8], int lane, float scale,
+                                              unsigned short (&h)[8]) {
+  float v[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = x[e] * s[e];
+  r4_fwht128_rows<8>(v, lane);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) h[e] = r4_f16_rn(v[e] * scale);
+}
+__device__ __forceinline__ float xq_amax8(const unsigned short (&h)[8]) {
+  float m = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) m = __builtin_fmaxf(m, __builtin_fabsf(r4_f16_to_f32(h[e])));
+  return m;
+}
+// 8 consecutive k (k % 8 == 0) of row r: two dwords, one per fragment half, 128 bytes apart in the A8 layout
+__device__ __forceinline__ void xq_store8(signed char* __restrict__ a8, int r, int k, int K, const unsigned short (&h)[8],
+                                          float sc) {
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    float v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = r4_f16_to_f32(h[4 * u + j]);
+    q_store4(a8, true, r, k + 4 * u, K, q_pack4(v, sc));
+  }
 }
 
-// per-(row, 128) scales: one wave per (row, kXqBlkU consecutive blocks), every load of its blocks issued before
-// the first transform (a block past the row re-reads the last one and is dropped); each block goes through a
-// wave-private LDS slot to reach q_blk_kernel's lane map (lane l: k = 2 l, 2 l + 1)
-constexpr int kXqBlkU = 4;
+// per-(row, 128) scales: a 16-lane row per (row, block); the four rows of a wave hold four consecutive blocks
 template <int SRC>
 __global__ __launch_bounds__(256) void xq_blk_kernel(R4XSrc src, int K, int nout, XqOut p, float scale) {
-  __shared__ unsigned short buf[4][128];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int nkb = K >> 7, ngr = (nkb + kXqBlkU - 1) / kXqBlkU;
+  const int nkb = K >> 7, ngr = (nkb + 3) >> 2;
   // workgroups are dealt to the 8 XCDs in turn: XCD x takes rows 32 x .. 32 x + 31 (two 16-row tiles of the A8
-  // layout), so the 8-byte pieces of one 256-byte A8 block are all written through one L2
+  // layout), so the pieces of one 256-byte A8 block are all written through one L2
   const int xcd = blockIdx.x & 7;
-  const long long j = (long long)(blockIdx.x >> 3) * 4 + w;
-  if (j >= 32LL * ngr) return;
-  const int row = 32 * xcd + (int)(j & 31), kbase = (int)(j >> 5) * kXqBlkU;
-  float x0[kXqBlkU], x1[kXqBlkU];
-  size_t k0[kXqBlkU];
+  const int j = (int)(blockIdx.x >> 3) * 4 + w;
+  const int row = 32 * xcd + (j & 31), kb = (j >> 5) * 4 + (lane >> 4);
+  if (j >= 32 * ngr || kb >= nkb) return;       // whole 16-lane rows leave together
+  const int k = 128 * kb + 8 * (lane & 15);
+  float x[8];
+  r4_xsrc_n<SRC, true, 8>(src, row, k, x);
+  float s[kXqMaxOut][8];
 #pragma unroll
-  for (int u = 0; u < kXqBlkU; ++u) {
-    k0[u] = (size_t)min(kbase + u, nkb - 1) * 128;
-    x0[u] = r4_xsrc<SRC, true>(src, row, (long long)k0[u] + lane);
-    x1[u] = r4_xsrc<SRC, true>(src, row, (long long)k0[u] + lane + 64);
-  }
-  for (int o = 0; o < nout; ++o) {
-    float s0[kXqBlkU], s1[kXqBlkU];
+  for (int o = 0; o < kXqMaxOut; ++o) r4_load_f32<8>(p.suh[o < nout ? o : 0] + k, s[o]);
 #pragma unroll
-    for (int u = 0; u < kXqBlkU; ++u) {
-      s0[u] = p.suh[o][k0[u] + lane];
-      s1[u] = p.suh[o][k0[u] + 64 + lane];
-    }
+  for (int o = 0; o < kXqMaxOut; ++o) {
+    if (o >= nout) break;
+    unsigned short h[8];
+    xq_transform8(x, s[o], lane, scale, h);
+    float amax = xq_amax8(h);
 #pragma unroll
-    for (int u = 0; u < kXqBlkU; ++u) {
-      if (kbase + u >= nkb) break;
-      unsigned short h0, h1;
-      xq_transform_s(x0[u], x1[u], s0[u], s1[u], lane, scale, h0, h1);
-      buf[w][lane] = h0;
-      buf[w][lane + 64] = h1;
-      // the wave reads what other lanes wrote: keep the read after the writes (and the next block's writes
-      // after this read) -- without the clobber the compiler hoists the read above the stores
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      const unsigned raw = *(const unsigned*)&buf[w][2 * lane];
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      const float v0 = r4_f16_to_f32((unsigned short)(raw & 0xFFFFu)), v1 = r4_f16_to_f32((unsigned short)(raw >> 16));
-      float amax = __builtin_fmaxf(__builtin_fabsf(v0), __builtin_fabsf(v1));
-#pragma unroll
-      for (int m = 32; m >= 1; m >>= 1) amax = __builtin_fmaxf(amax, __shfl_xor(amax, m, 64));
-      const float sc = q_scale(amax);
-      const int kb = kbase + u;
-      if (lane == 0) p.sa[o][(size_t)kb * 256 + row] = sc;
-      const unsigned q01 = ((unsigned)q_one(v0, sc) & 0xFFu) | (((unsigned)q_one(v1, sc) & 0xFFu) << 8);
-      const unsigned q23 = (unsigned)__shfl_xor((int)q01, 1, 64);
-      if ((lane & 1) == 0) q_store4(p.a8[o], true, row, (int)k0[u] + 2 * lane, K, q01 | (q23 << 16));
-    }
+    for (int m = 1; m <= 8; m <<= 1) amax = __builtin_fmaxf(amax, r4_xor_lane(amax, m));
+    const float sc = q_scale(amax);
+    if ((lane & 15) == 0) p.sa[o][(size_t)kb * 256 + row] = sc;
+    xq_store8(p.a8[o], row, k, K, h, sc);
   }
 }
 
-// one scale per row: a workgroup (kXqRowWaves waves) per row transforms every block into LDS (f16, [nout][K]),
-// takes the row's amax, then quantizes like q_row_kernel. 16 waves per row: with 4 (one per SIMD) each wave walked
-// its blocks one memory round trip at a time (K 17408: 26 us per launch)
+// one scale per row: a workgroup (kXqRowWaves waves, 64 blocks at a time) per row keeps its transformed f16 values in LDS
+// ([nout][K], each lane reading back its own 16 bytes), takes the row's amax, then quantizes. 16 waves per row: with 4
+// (one per SIMD) each wave walked its blocks one memory round trip at a time (K 17408: 26 us per launch)
 constexpr int kXqRowWaves = 16;
 template <int SRC>
 __global__ __launch_bounds__(64 * kXqRowWaves) void xq_row_kernel(R4XSrc src, int K, int nout, XqOut p, float scale) {
-  extern __shared__ unsigned short rowbuf[];
+  extern __shared__ r4u4 rowbuf[];
   __shared__ float red[kXqMaxOut][kXqRowWaves];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  // XCD x (workgroups are dealt to the 8 XCDs in turn) takes rows 32 x .. 32 x + 31: the 8-byte pieces of one
-  // 256-byte A8 block (16 rows) are then all written through one L2
-  const int row = 32 * (blockIdx.x & 7) + (blockIdx.x >> 3), nkb = K >> 7;
+  // XCD x (workgroups are dealt to the 8 XCDs in turn) takes rows 32 x .. 32 x + 31: the pieces of one 256-byte A8
+  // block are then all written through one L2
+  const int row = 32 * (blockIdx.x & 7) + (blockIdx.x >> 3), nch = K >> 3;   // 8-element chunks, one per lane
   float amax[kXqMaxOut] = {0.f, 0.f, 0.f};
-  // kXqRowU blocks per pass, all their loads issued first (a block past the row re-reads the last one and is
-  // dropped), so a wave waits for one memory round trip per pass instead of one per block
-  constexpr int kXqRowU = 3;
-  for (int kb = w; kb < nkb; kb += kXqRowU * kXqRowWaves) {
-    float x0[kXqRowU], x1[kXqRowU];
-    size_t k0[kXqRowU];
+  for (int c = threadIdx.x; c < nch; c += 64 * kXqRowWaves) {   // 16 divides nch: whole 16-lane rows
+    float x[8];
+    r4_xsrc_n<SRC, true, 8>(src, row, 8LL * c, x);
+    float s[kXqMaxOut][8];
 #pragma unroll
-    for (int u = 0; u < kXqRowU; ++u) {
-      const int b = min(kb + u * kXqRowWaves, nkb - 1);
-      k0[u] = (size_t)b * 128;
-      x0[u] = r4_xsrc<SRC, true>(src, row, (long long)k0[u] + lane);
-      x1[u] = r4_xsrc<SRC, true>(src, row, (long long)k0[u] + lane + 64);
-    }
+    for (int o = 0; o < kXqMaxOut; ++o) r4_load_f32<8>(p.suh[o < nout ? o : 0] + 8 * c, s[o]);
 #pragma unroll
     for (int o = 0; o < kXqMaxOut; ++o) {
       if (o >= nout) break;
-      float s0[kXqRowU], s1[kXqRowU];
-#pragma unroll
-      for (int u = 0; u < kXqRowU; ++u) {
-        s0[u] = p.suh[o][k0[u] + lane];
-        s1[u] = p.suh[o][k0[u] + 64 + lane];
-      }
-#pragma unroll
-      for (int u = 0; u < kXqRowU; ++u) {
-        unsigned short h0, h1;
-        xq_transform_s(x0[u], x1[u], s0[u], s1[u], lane, scale, h0, h1);
-        if (kb + u * kXqRowWaves < nkb) {
-          rowbuf[(size_t)o * K + k0[u] + lane] = h0;
-          rowbuf[(size_t)o * K + k0[u] + lane + 64] = h1;
-          amax[o] = __builtin_fmaxf(amax[o], __builtin_fmaxf(__builtin_fabsf(r4_f16_to_f32(h0)),
-                                                             __builtin_fabsf(r4_f16_to_f32(h1))));
-        }
-      }
+      unsigned short h[8];
+      xq_transform8(x, s[o], lane, scale, h);
+      rowbuf[(size_t)o * nch + c] = (r4u4){h[0] | (unsigned)h[1] << 16, h[2] | (unsigned)h[3] << 16,
+                                           h[4] | (unsigned)h[5] << 16, h[6] | (unsigned)h[7] << 16};
+      amax[o] = __builtin_fmaxf(amax[o], xq_amax8(h));
     }
   }
 #pragma unroll
   for (int o = 0; o < kXqMaxOut; ++o) {
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) amax[o] = __builtin_fmaxf(amax[o], __shfl_xor(amax[o], m, 64));
+    for (int m = 32; m >= 1; m >>= 1) amax[o] = __builtin_fmaxf(amax[o], r4_xor_lane(amax[o], m));
     if (lane == 0) red[o][w] = amax[o];
   }
   __syncthreads();
@@ -248,11 +226,12 @@ __global__ __launch_bounds__(64 * kXqRowWaves) void xq_row_kernel(R4XSrc src, in
     for (int i = 1; i < kXqRowWaves; ++i) m = __builtin_fmaxf(m, red[o][i]);
     const float s = q_scale(m);
     if (threadIdx.x == 0) p.sa[o][row] = s;
-    for (int k = threadIdx.x * 4; k < K; k += 4 * 64 * kXqRowWaves) {
-      float v[4];
+    for (int c = threadIdx.x; c < nch; c += 64 * kXqRowWaves) {
+      const r4u4 raw = rowbuf[(size_t)o * nch + c];
+      unsigned short h[8];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = r4_f16_to_f32(rowbuf[(size_t)o * K + k + j]);
-      q_store4(p.a8[o], true, row, k, K, q_pack4(v, s));
+      for (int e = 0; e < 8; ++e) h[e] = (unsigned short)(raw[e >> 1] >> (16 * (e & 1)));
+      xq_store8(p.a8[o], row, 8 * c, K, h, s);
     }
   }
 }
@@ -269,7 +248,7 @@ void xq_launch(bool row_scale, const R4XSrc& src, int64_t K, int nout, const XqO
     if (lds > 64 * 1024) r4d::allow_lds((const void*)xq_row_kernel<SRC>, lds_set, entry);
     hipLaunchKernelGGL((xq_row_kernel<SRC>), dim3(256), dim3(64 * kXqRowWaves), lds, st, src, (int)K, nout, p, scale);
   } else {
-    const long long waves = 256LL * ((K / 128 + kXqBlkU - 1) / kXqBlkU);
+    const long long waves = 256LL * ((K / 128 + 3) / 4);
     hipLaunchKernelGGL((xq_blk_kernel<SRC>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st, src, (int)K, nout,
                        p, scale);
   }

@@ -73,6 +73,12 @@ typedef unsigned r4u4 __attribute__((ext_vector_type(4)));
 typedef unsigned r4u2 __attribute__((ext_vector_type(2)));
 typedef float r4f2 __attribute__((ext_vector_type(2)));
 typedef int r4i4 __attribute__((ext_vector_type(4)));
+// 16- and 8-byte accesses at the element type's own alignment: callers' tensors need no more than that
+typedef unsigned r4u4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef unsigned r4u2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+typedef unsigned r4u1_a2 __attribute__((aligned(2)));
+typedef float r4f4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float r4f2_a4 __attribute__((ext_vector_type(2), aligned(4)));
 
 #define R4_WAVE 64
 
@@ -160,6 +166,63 @@ __device__ __forceinline__ float r4_xsrc(const R4XSrc& s, long long row, long lo
   } else {
     const float a = r4_bf16_to_f32(s.p0[i]), g = r4_bf16_to_f32(s.p1[i]);
     return r4_bf16_to_f32(r4_bf16_rn(a * r4_sigmoid(g)));
+  }
+}
+
+// x[row][k .. k + E - 1] (E = 2 or 8) with one load per array that needs no more than the elements' own alignment
+template <int E>
+__device__ __forceinline__ void r4_load_u16(const unsigned short* p, unsigned (&d)[E / 2]) {
+  if constexpr (E == 8) {
+    const r4u4 v = *(const r4u4_a2*)p;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d[i] = v[i];
+  } else {
+    d[0] = *(const r4u1_a2*)p;
+  }
+}
+template <int SRC, bool BF16, int E>
+__device__ __forceinline__ void r4_xsrc_n(const R4XSrc& s, long long row, long long k, float (&x)[E]) {
+  const long long i = row * s.ld + k;
+  unsigned a[E / 2], b[E / 2];
+  r4_load_u16<E>(s.p0 + i, a);
+  if constexpr (SRC == R4_SRC_SILU) r4_load_u16<E>(s.p0 + i + s.off, b);
+  if constexpr (SRC == R4_SRC_GATE) r4_load_u16<E>(s.p1 + i, b);
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const unsigned short ha = (unsigned short)(a[e >> 1] >> (16 * (e & 1)));
+    if constexpr (SRC == R4_SRC_X) {
+      x[e] = BF16 ? r4_bf16_to_f32(ha) : r4_f16_to_f32(ha);
+    } else {
+      const float v = r4_bf16_to_f32(ha), w = r4_bf16_to_f32((unsigned short)(b[e >> 1] >> (16 * (e & 1))));
+      x[e] = r4_bf16_to_f32(r4_bf16_rn_sel(SRC == R4_SRC_SILU ? v * r4_sigmoid(v) * w : v * r4_sigmoid(w)));
+    }
+  }
+}
+// E floats at 4-byte alignment
+template <int E>
+__device__ __forceinline__ void r4_load_f32(const float* p, float (&d)[E]) {
+  if constexpr (E == 2) {
+    const r4f2 v = *(const r4f2_a4*)p;
+    d[0] = v[0];
+    d[1] = v[1];
+  } else {
+#pragma unroll
+    for (int i = 0; i < E; i += 4) {
+      const r4f4 v = *(const r4f4_a4*)(p + i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) d[i + e] = v[e];
+    }
+  }
+}
+// E 16-bit values at 2-byte alignment
+template <int E>
+__device__ __forceinline__ void r4_store_u16(unsigned short* p, const unsigned (&h)[E]) {
+  if constexpr (E == 8) {
+    *(r4u4_a2*)p = (r4u4){h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16};
+  } else if constexpr (E == 4) {
+    *(r4u2_a2*)p = (r4u2){h[0] | h[1] << 16, h[2] | h[3] << 16};
+  } else {
+    *(r4u1_a2*)p = h[0] | h[1] << 16;
   }
 }
 
@@ -277,14 +340,14 @@ __device__ __forceinline__ int r4_lane_word(int c, int i) {
 // 120-131): for lg < 6 the partner is lane l ^ 2^lg and the lower index keeps a + b, the upper takes
 // a - b (= partner - own); lg = 6 pairs the two registers.
 // v of lane l ^ mask (mask a power of two below 64, a compile-time constant after unrolling). Masks 1-8 are
-// DPP moves inside a row of 16 lanes (ALU latency; 4 and 8 as two mirrors: (l ^ 7) ^ 3 = l ^ 4, (l ^ 15) ^ 7
-// = l ^ 8), 16 a ds_swizzle inside 32 lanes, 32 a ds_bpermute. Pure data movement: the values are unchanged.
+// DPP moves inside a row of 16 lanes (ALU latency; 4 as two mirrors: (l ^ 7) ^ 3 = l ^ 4; 8 a rotation by 8), 16 a
+// ds_swizzle inside 32 lanes, 32 a ds_bpermute. Pure data movement: the values are unchanged.
 __device__ __forceinline__ int r4_xor_lane_i(int v, int mask) {
   switch (mask) {
     case 1: return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true);     // quad_perm [1, 0, 3, 2]
     case 2: return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true);     // quad_perm [2, 3, 0, 1]
     case 4: return __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, true), 0x1B, 0xF, 0xF, true);
-    case 8: return __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(v, 0x140, 0xF, 0xF, true), 0x141, 0xF, 0xF, true);
+    case 8: return __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, true);    // row_ror:8
     case 16: return __builtin_amdgcn_ds_swizzle(v, (16 << 10) | 0x1F);  // bit mode, xor 16 inside 32 lanes
     default: return __shfl_xor(v, mask, R4_WAVE);
   }
@@ -321,6 +384,40 @@ __device__ __forceinline__ void r4_fwht128_wave_pairs(float& v0, float& v1, int 
     const bool upper = (lane & hm) != 0;
     v0 = upper ? p0 - v0 : v0 + p0;
     v1 = upper ? p1 - v1 : v1 + p1;
+  }
+}
+
+// The same transform with E = 8, 4 or 2 adjacent elements per lane: lane i of a row of 128 / E lanes holds elements E i ..
+// E i + E - 1, so the first log2 E stages are in registers and the rest exchange with lanes i ^ 1, 2, 4, 8 (DPP), i ^ 16
+// and i ^ 32 (v_permlane16_swap, v_permlane32_swap): no stage goes through the LDS crossbar, and a wave transforms E / 2
+// rows at once. Each stage is own * (+-1) + partner: the sign flips for the upper index (a - b is partner - own), so
+// every element sees the same fp32 operations in the same order as in r4_fwht128_wave.
+template <int E>
+__device__ __forceinline__ void r4_fwht128_rows(float (&v)[E], int lane) {
+#pragma unroll
+  for (int b = 1; b < E; b <<= 1)
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      if ((e & b) == 0) {
+        const float x = v[e], y = v[e | b];
+        v[e] = x + y;
+        v[e | b] = x - y;
+      }
+#pragma unroll
+  for (int hm = 1; hm < 128 / E; hm <<= 1) {
+    const unsigned sg = (lane & hm) ? 0x80000000u : 0u;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const unsigned u = __builtin_bit_cast(unsigned, v[e]);
+      if (hm <= 8) {
+        v[e] = __builtin_bit_cast(float, u ^ sg) + r4_xor_lane(v[e], hm);
+      } else {
+        // the swap of a value with itself: [0] the lower half's value in both halves of an exchange, [1] the upper's
+        const auto s = hm == 16 ? __builtin_amdgcn_permlane16_swap(u, u, false, false)
+                                : __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        v[e] = __builtin_bit_cast(float, (unsigned)s[0]) + __builtin_bit_cast(float, (unsigned)s[1] ^ sg);
+      }
+    }
   }
 }
 

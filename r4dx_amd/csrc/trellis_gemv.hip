@@ -14,57 +14,11 @@
 // (ticket) sums them in a fixed order and finishes: FWHT-128 in fp32 in the reference's stage order,
 // * svh, * out_scale, one bf16 rounding. A row's bits depend on (K, N, KB, SKG, SK) only -- never on M,
 // on the pairs per workgroup or on the other rows -- so decode rows equal verify rows for every M <= 64.
-#include "r4d_dev.h"
 #include "r4d_host.h"
+#include "tq_common.h"
 #include "r4d_mi355x.h"
 
 namespace {
-
-template <int KB>
-struct Words {
-  unsigned w[KB + 1];   // [0] history, [1..KB] own words
-};
-
-#define R4_RSRC_FLAGS 0x00020000
-typedef __amdgpu_buffer_rsrc_t r4_rsrc;
-__device__ __forceinline__ r4_rsrc r4_make_rsrc(const void* p, unsigned bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, (int)bytes, R4_RSRC_FLAGS);
-}
-
-// Byte offsets, inside a (pair, k-tile) block, of the lane's own words (KB c .. KB c + KB - 1 of tile t)
-// and history word (KB c - 1 mod 8 KB); block q of a step sits q * 64 KB bytes further.
-template <int KB>
-struct LaneWords {
-  unsigned own, hist;
-  __device__ __forceinline__ LaneWords(int q, int t, int c) {
-    const unsigned tile = (unsigned)(q * 16 * KB + t * 8 * KB);
-    own = (tile + KB * c) * 4u;
-    hist = (tile + (KB * c - 1 + 8 * KB) % (8 * KB)) * 4u;
-  }
-};
-
-// Cache policy of the weight loads: nontemporal (each word is read once per launch; measured ~2 % faster
-// per step than the default policy).
-constexpr int kWeightPolicy = 2;
-
-// One step's words of this lane from the slice buffer at step byte offset so (out of range -> 0).
-template <int KB, bool HIST = true>
-__device__ __forceinline__ void load_words(Words<KB>& s, r4_rsrc r, const LaneWords<KB>& lw, unsigned so) {
-  // one wide load per lane where the KB words allow it (buffer loads need dword alignment only): KB 4 one dwordx4,
-  // KB 5 a dwordx4 and a dword, KB 3 a dwordx3 -- not KB dword loads, each of which would touch every line of the step
-  if constexpr (KB == 4 || KB == 5) {
-    const r4u4 v = __builtin_bit_cast(r4u4, __builtin_amdgcn_raw_buffer_load_b128(r, lw.own + so, 0, kWeightPolicy));
-    s.w[1] = v[0]; s.w[2] = v[1]; s.w[3] = v[2]; s.w[4] = v[3];
-    if constexpr (KB == 5) s.w[5] = __builtin_amdgcn_raw_buffer_load_b32(r, lw.own + so + 16, 0, kWeightPolicy);
-  } else if constexpr (KB == 3) {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b96(r, lw.own + so, 0, kWeightPolicy);
-    s.w[1] = v[0]; s.w[2] = v[1]; s.w[3] = v[2];
-  } else {
-#pragma unroll
-    for (int i = 0; i < KB; ++i) s.w[1 + i] = __builtin_amdgcn_raw_buffer_load_b32(r, lw.own + so + 4 * i, 0, kWeightPolicy);
-  }
-  if constexpr (HIST) s.w[0] = __builtin_amdgcn_raw_buffer_load_b32(r, lw.hist + so, 0, kWeightPolicy);
-}
 
 // A row's two fragments (h = 0, 1) of one k-tile from the row buffer at byte offset off:
 // k 16kt + {0..3, 8..11} and {4..7, 12..15}.
@@ -92,31 +46,12 @@ __device__ __forceinline__ void load_words_ptr(Words<KB>& s, const unsigned* __r
 // balance the VALU-bound decode over the CUs (measured better on gfx950 than a persistent grid).
 // Weights are prefetched PF steps ahead (a step is 4 k-tiles = one dwordx4 per lane) and issued before
 // A is staged in LDS.
-constexpr int kRedParts = 8;         // the final slice sum is 8 interleaved runs, added in order
-constexpr int kRedRows = 4;          // rows of the final slice sum per pass (8 measured slower at M = 8: LDS)
-
-// n / d for the staging loops' row split (d = M <= 64, n below 2^20): one high multiply by the launch-uniform
-// floor(2^32 / d) + 1, exact whenever n d < 2^32 (the error term n e / (d 2^32), 0 < e <= d, stays below 1 / d);
-// d = 1 (whose multiplier would need 33 bits) is marked by 0 and returns n.
-// The multipliers for d = 0..64 as a constant table (d = 0 unused): a scalar load of the launch's M instead of a 64-bit
-// division formed with VALU ops in every wave.
-struct R4DivMagic {
-  unsigned m[65];
-  constexpr R4DivMagic() : m() {
-    for (unsigned d = 1; d <= 64; ++d) m[d] = d == 1u ? 0u : (unsigned)(0x100000000ull / d) + 1u;
-  }
-};
-__constant__ constexpr R4DivMagic kR4DivMagic{};
-__device__ __forceinline__ unsigned r4_div_magic(unsigned d) { return kR4DivMagic.m[d]; }
-__device__ __forceinline__ int r4_div_by(int n, unsigned magic) {
-  return magic ? (int)__umulhi((unsigned)n, magic) : n;
-}
-
 // XF > 0: A0 is the raw input x [M][K] (XF 1: f16, 2: bf16) and the workgroup stages its own slice of the
 // transformed A = f16(FWHT128(fp32(x) * suh) * xscale) (suh of the group's column part) straight into LDS --
 // the arithmetic of r4dx_trellis_input_*, so A is bit-identical to the unfused path's.
+// The decode forms (one row tile, A in LDS) ask for 6 waves per SIMD: their register need lies just above that budget.
 template <int KB, int MT, int NPW, int SK, bool ALDS, int XF, bool WQ = false>
-__global__ __launch_bounds__(64 * NPW * SK) void tq_gemv_kernel(
+__global__ __launch_bounds__(64 * NPW * SK, MT == 1 && ALDS && SK == 4 && XF == 0 && !WQ ? 6 : 1) void tq_gemv_kernel(
     const R4AParts ap,
     const unsigned* __restrict__ W, const float* __restrict__ svh, void* __restrict__ Cv,
     float* __restrict__ ws, unsigned* __restrict__ tickets, int M, int K, int N, int SKG, int full,
@@ -156,14 +91,9 @@ __global__ __launch_bounds__(64 * NPW * SK) void tq_gemv_kernel(
   const unsigned mmag = r4_div_magic((unsigned)M);
 
   // LDS: the A slice (ALDS) + its zero block while the k loop runs; after it (every wave past the barrier that ends
-  // the loop), the same bytes hold [SK - 1 partial accumulators per pair] [M x 128 sums] [8 x 4 x 128 reduce runs]
-  // [flag]. The launch asks for the larger of the two.
+  // the loop), the same bytes hold the unit's end (tq_end_lds). The launch asks for the larger of the two.
   r4u4* alds = lds_raw;
-  float* part_acc = (float*)lds_raw;                                 // [(SK-1) * NPW][8 MT][64]
-  float* red = part_acc + (size_t)(SK - 1) * NPW * 8 * MT * 64;      // [M][128]
-  float* runs = red + (size_t)M * 128;                               // [8][4][128]
-  const int red_rows = min(kRedRows, M);      // rows per finish pass (the LDS holds no more)
-  int* flag = (int*)(runs + (size_t)kRedParts * red_rows * 128);
+  float* part_acc = (float*)lds_raw;
 
   const unsigned* __restrict__ wpair = W + ((size_t)pair * KT + kt0) * BLK;
   const r4_rsrc wr = r4_make_rsrc(wpair, (unsigned)ktw * BLK * 4u);
@@ -398,184 +328,15 @@ __global__ __launch_bounds__(64 * NPW * SK) void tq_gemv_kernel(
 
   // The A slice is dead once every wave has left the loop: the combine, the sums and the reduce runs reuse its bytes.
   if constexpr (ALDS) __syncthreads();
-  // Combine the SK waves of each pair in k order (ks = 0, 1, ...) into wave ks = 0.
-  if constexpr (SK > 1) {
-    if (ks > 0) {
-      float* dst = part_acc + ((size_t)((ks - 1) * NPW + pl) * 8 * MT) * 64;
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int f = 0; f < 2; ++f)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) dst[((i * 2 + f) * 4 + j) * 64 + lane] = acc[i][f][j];
-    }
-    __syncthreads();
-    if (ks == 0) {
-#pragma unroll
-      for (int s = 1; s < SK; ++s) {
-        const float* src = part_acc + ((size_t)((s - 1) * NPW + pl) * 8 * MT) * 64;
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-          for (int f = 0; f < 2; ++f)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][f][j] += src[((i * 2 + f) * 4 + j) * 64 + lane];
-      }
-    }
-  }
+  tq_combine<MT, NPW, SK>(acc, part_acc, pl, ks, lane);
 
   if (probe) {
     clk[2] = __builtin_amdgcn_s_memtime();
     clk[3] = __builtin_amdgcn_s_memrealtime();
   }
 
-  // Lane l of wave (pl, ks = 0) holds rows 16 i + 4 (l >> 4) + j of column slot nb = l & 15 of
-  // fragment cs: true column 32 pair + 16 (nb >> 3) + (nb & 7) + 8 cs.
-  const int nb = lane & 15, rq = lane >> 4;
-  const int gcol0 = (pair & 3) * 32 + 16 * (nb >> 3) + (nb & 7);   // inside the group
-  float* Cf = (float*)Cv;
-  unsigned short* Cb = (unsigned short*)Cv;
-  const int n0 = group * 128;
-  const bool in_block = NPW == 4 && SKG == 1;   // the workgroup holds its whole group
-
-  if (SKG == 1 && !full) {
-    if (ks == 0) {
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int r = 16 * i + 4 * rq + j;
-          if (r < M) {
-            Cf[(size_t)r * N + n0 + gcol0] = acc[i][0][j];
-            Cf[(size_t)r * N + n0 + gcol0 + 8] = acc[i][1][j];
-          }
-        }
-    }
-    return;
-  }
-  if (in_block) {
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int r = 16 * i + 4 * rq + j;
-        if (r < M) {
-          red[r * 128 + gcol0] = acc[i][0][j];
-          red[r * 128 + gcol0 + 8] = acc[i][1][j];
-        }
-      }
-    __syncthreads();
-  } else {
-    if (ks == 0) {
-      float* wsy = ws + (size_t)ky * M * N;
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int r = 16 * i + 4 * rq + j;
-          if (r < M) {
-            r4_store_coherent(&wsy[(size_t)r * N + n0 + gcol0], acc[i][0][j]);
-            r4_store_coherent(&wsy[(size_t)r * N + n0 + gcol0 + 8], acc[i][1][j]);
-          }
-        }
-    }
-    if (!r4_ticket_last(&tickets[group * R4_TICKET_WORDS], (unsigned)(SKG * (4 / NPW)), flag)) return;
-    // Sum the SKG slices: run p (0..7) adds slices p, p + 8, ... in order; the 8 runs are then added
-    // in order 0..7 -- the same arithmetic for every element whatever M is. kRedRows rows at a time
-    // (bounded LDS); the finished sums land in red[r][128] for the epilogue.
-    // SKG <= 64, so one batch of 8 loads (slices p, p + 8, ..., p + 56) covers a run. The loads are
-    // coherent (sc1) buffer loads over ws: a slice past SKG or an item past the end reads past the buffer
-    // and returns 0, so every thread issues all loads of its kFinItems items at once, with no branches.
-    const unsigned sy4 = (unsigned)M * (unsigned)N * 4u;
-    const r4_rsrc wsr = r4_make_rsrc(ws, (unsigned)SKG * sy4);
-    if (SKG <= kRedParts) {
-      // At most one slice per run (every planned split): each thread sums whole elements -- run p is 0.f + slice p,
-      // the runs are added in order and the empty ones (p >= SKG) add +0.f, which the one addition below stands for
-      // (adding +0.f again changes nothing) -- with its SKG loads issued at once: the same bits as the general form
-      // below, without its loads of absent slices and its second pass through LDS.
-      constexpr int kFinE = 2;   // elements per thread per pass
-      for (int e0 = (int)threadIdx.x; e0 < M * 128; e0 += kFinE * NT) {
-        float tv[kFinE][kRedParts];
-#pragma unroll
-        for (int it = 0; it < kFinE; ++it) {
-          const int e = e0 + it * NT;
-          const unsigned off = e < M * 128 ? ((unsigned)(e >> 7) * (unsigned)N + (unsigned)(n0 + (e & 127))) * 4u : 0xFFFFFFF0u;
-#pragma unroll
-          for (int p = 0; p < kRedParts; ++p)
-            if (p < SKG)
-              tv[it][p] = __builtin_bit_cast(
-                  float, __builtin_amdgcn_raw_buffer_load_b32(wsr, off == 0xFFFFFFF0u ? off : off + (unsigned)p * sy4, 0, 16));
-        }
-#pragma unroll
-        for (int it = 0; it < kFinE; ++it) {
-          const int e = e0 + it * NT;
-          float v = 0.f + tv[it][0];
-#pragma unroll
-          for (int p = 1; p < kRedParts; ++p)
-            if (p < SKG) v += 0.f + tv[it][p];
-          if (SKG < kRedParts) v += 0.f;
-          if (e < M * 128) {
-            if (full) red[e] = v;
-            else Cf[(size_t)(e >> 7) * N + n0 + (e & 127)] = v;
-          }
-        }
-      }
-      __syncthreads();
-      if (!full) return;
-    } else {
-    constexpr int kFinItems = 4;
-    for (int r0 = 0; r0 < M; r0 += red_rows) {
-      const int rows = min(red_rows, M - r0);
-      const int items = kRedParts * rows * 128;
-      for (int b0 = 0; b0 < items; b0 += kFinItems * NT) {
-        float tv[kFinItems][8];
-#pragma unroll
-        for (int it = 0; it < kFinItems; ++it) {
-          const int idx = b0 + it * NT + (int)threadIdx.x;
-          const int p = idx / (rows * 128), e = idx - p * rows * 128;
-          const unsigned off = idx < items ? (unsigned)p * sy4 + ((unsigned)(r0 + (e >> 7)) * (unsigned)N + (unsigned)(n0 + (e & 127))) * 4u
-                                           : 0xFFFFFFF0u;
-#pragma unroll
-          for (int u = 0; u < 8; ++u) {
-            const unsigned ou = off + (unsigned)u * (unsigned)kRedParts * sy4;
-            const unsigned o = (off == 0xFFFFFFF0u || ou < off) ? 0xFFFFFFF0u : ou;   // wrap-safe
-            tv[it][u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wsr, o, 0, 16));
-          }
-        }
-#pragma unroll
-        for (int it = 0; it < kFinItems; ++it) {
-          const int idx = b0 + it * NT + (int)threadIdx.x;
-          if (idx < items) {
-            const int p = idx / (rows * 128), e = idx - p * rows * 128;
-            float v = 0.f;
-#pragma unroll
-            for (int u = 0; u < 8; ++u) v += tv[it][u];
-            runs[(size_t)p * red_rows * 128 + e] = v;
-          }
-        }
-      }
-      __syncthreads();
-      for (int e = threadIdx.x; e < rows * 128; e += NT) {
-        float v = runs[e];
-#pragma unroll
-        for (int p = 1; p < kRedParts; ++p) v += runs[(size_t)p * red_rows * 128 + e];
-        if (full) red[(size_t)r0 * 128 + e] = v;
-        else Cf[(size_t)(r0 + (e >> 7)) * N + n0 + (e & 127)] = v;
-      }
-      __syncthreads();
-    }
-    if (!full) return;
-    }
-  }
-  // The epilogue: one wave per row, the group's 128 sums as (lane, lane + 64).
-  const float sv0 = svh[n0 + lane], sv1 = svh[n0 + lane + 64];
-  for (int r = wave; r < M; r += NW) {
-    float v0 = red[r * 128 + lane], v1 = red[r * 128 + lane + 64];
-    r4_fwht128_wave(v0, v1, lane);
-    const float y0 = v0 * sv0, y1 = v1 * sv1;
-    Cb[(size_t)r * N + n0 + lane] = r4_bf16_rn(y0 * out_scale);
-    Cb[(size_t)r * N + n0 + lane + 64] = r4_bf16_rn(y1 * out_scale);
-  }
+  const TqOut out{svh, Cv, ws, tickets, M, N, SKG, full, out_scale};
+  tq_finish<MT, NPW, SK>(acc, (unsigned char*)lds_raw, out, group, pair, ks, ky);
 }
 
 // One wave per (tile pair, 4-k-tile step): every lane decodes its 32 weights with the GEMM's own
@@ -654,12 +415,10 @@ __global__ __launch_bounds__(256) void tq_wscale_kernel(const unsigned* __restri
 
 // Dynamic LDS of one launch.
 size_t gemv_ktl_pad(int SK, int ktw) { return (size_t)SK * ((((ktw + 3) >> 2) + SK - 1) / SK) * 4; }
-// The A slice (ALDS) and, after the k loop, in the same bytes: the partial accumulators, the sums, the reduce runs and
-// the flag.
+// The A slice (ALDS) and, after the k loop, in the same bytes: the unit's end.
 size_t gemv_lds(int MT, int NPW, int SK, bool alds, int ktw, int M) {
   const size_t a = alds ? gemv_ktl_pad(SK, ktw) * M * 32 + 32 : 0;
-  const size_t tail = (size_t)(SK - 1) * NPW * 8 * MT * 64 * 4 +
-                      (size_t)(M + kRedParts * (M < kRedRows ? M : kRedRows)) * 128 * 4 + 16;
+  const size_t tail = tq_end_lds(MT, NPW, SK, M);
   return a > tail ? a : tail;
 }
 constexpr size_t kAldsMax = 48 * 1024;   // A slices up to this many bytes are staged in LDS

@@ -3,9 +3,8 @@
 // 63-100 and tests/kernels/trellis_ref.hpp:150-169):
 //   out[o][m, k] = f16( fp32( FWHT128( fp32(x[m, :]) * suh[o][:] )[k] * scale ) ),  scale = float(2^s / sqrt(128))
 // per 128-block, fp32 butterflies in the reference's stage order, the product x * suh and the final
-// product each rounded to fp32, then ONE rounding to f16. One wave64 per (128-block, row): lane l
-// holds elements l and l + 64. Also r4dx_fwht128_f32 (kernels.h:192-197), and the fused producers
-// (kernels.h:130-147; trellis_transform.hip:100-170): the transform of bf16(silu(gate) * up) or of
+// product each rounded to fp32, then ONE rounding to f16. Also r4dx_fwht128_f32 (kernels.h:192-197), and the
+// fused producers (kernels.h:130-147; trellis_transform.hip:100-170): the transform of bf16(silu(gate) * up) or of
 // bf16(attn_out * sigmoid(gate)) in one launch, each element the bf16 value the producer kernel
 // (r4dx_silu_mul_wide_bf16, kernels.h:90-91; r4dx_model_attn_gate_mul_bf16, attn_kernels.h:30-31, also
 // here) would have stored, so the result is byte-identical to the producer followed by the transform.
@@ -21,33 +20,52 @@ struct OutPtrs {
   unsigned short* out[kMaxOut];
 };
 
-template <int SRC, bool BF16>
-__global__ __launch_bounds__(64) void tq_input_kernel(R4XSrc src, int64_t K, int nout, OutPtrs p, float scale) {
-  const int lane = threadIdx.x;
-  const int64_t k0 = (int64_t)blockIdx.x * 128;
-  const int64_t row = blockIdx.y;
-  const float x0 = r4_xsrc<SRC, BF16>(src, row, k0 + lane);
-  const float x1 = r4_xsrc<SRC, BF16>(src, row, k0 + lane + 64);
+// 128 / E lanes per (row, 128-block), E adjacent elements per lane (r4_fwht128_rows): wide loads of x and stores of A, and
+// a Hadamard that stays in registers and DPP moves. A wave takes E / 2 consecutive items of the row-major item list.
+template <int SRC, bool BF16, int E>
+__global__ __launch_bounds__(256) void tq_input_kernel(R4XSrc src, long long K, int row0, int items, int nout, OutPtrs p,
+                                                       float scale) {
+  const int lane = threadIdx.x & 63;
+  const int id = (int)((blockIdx.x * blockDim.x + threadIdx.x) / (128 / E));
+  if (id >= items) return;                      // the lanes of an item leave together
+  const int nkb = (int)(K >> 7), rl = id / nkb;
+  const long long row = row0 + rl, k = 128LL * (id - rl * nkb) + E * (lane & (128 / E - 1));
+  float x[E];
+  r4_xsrc_n<SRC, BF16, E>(src, row, k, x);
   // every output's suh requested up front (an absent output reads the first one's): one memory round trip for the
   // wave instead of one per output
-  float s0[kMaxOut], s1[kMaxOut];
+  float s[kMaxOut][E];
+#pragma unroll
+  for (int o = 0; o < kMaxOut; ++o) r4_load_f32<E>(p.suh[o < nout ? o : 0] + k, s[o]);
 #pragma unroll
   for (int o = 0; o < kMaxOut; ++o) {
-    const float* sp = p.suh[o < nout ? o : 0];
-    s0[o] = sp[k0 + lane];
-    s1[o] = sp[k0 + lane + 64];
+    if (o >= nout) break;
+    float v[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = x[e] * s[o][e];
+    r4_fwht128_rows<E>(v, lane);
+    unsigned h[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) h[e] = r4_f16_rn(v[e] * scale);
+    r4_store_u16<E>(p.out[o] + row * K + k, h);
   }
-  // every output computed (an absent one's work is discarded), so the loads above stay ahead of all of it
-#pragma unroll
-  for (int o = 0; o < kMaxOut; ++o) {
-    float v0 = x0 * s0[o];
-    float v1 = x1 * s1[o];
-    r4_fwht128_wave(v0, v1, lane);
-    if (o < nout) {
-      unsigned short* dst = p.out[o] + row * K + k0;
-      dst[lane] = r4_f16_rn(v0 * scale);
-      dst[lane + 64] = r4_f16_rn(v1 * scale);
-    }
+}
+// E = 8 is the form with the fewest instructions per element; a launch too small to give every SIMD a wave of it (fewer
+// than 4096 items) is latency-bound and takes E = 2 in one-wave workgroups: a quarter of each lane's serial work, four
+// times the waves (one row of 17408 through silu: 4.0 us at best at E = 8, 2.6 at E = 2; 256 rows: 10.6 us at E = 8, 13.7 at two
+// elements per lane, all stages through the LDS crossbar).
+constexpr int64_t kWideItems = 4096;
+template <int SRC, bool BF16>
+void input_launch(const R4XSrc& src, int64_t rows, int64_t K, int nout, const OutPtrs& p, float scale, hipStream_t st) {
+  const int64_t nkb = K / 128, most = nkb < (1 << 25) ? (1 << 25) / nkb : 1;   // rows whose lanes a 32-bit index holds
+  for (int64_t r0 = 0; r0 < rows; r0 += most) {
+    const int64_t items = (rows - r0 < most ? rows - r0 : most) * nkb;
+    if (items < kWideItems)
+      hipLaunchKernelGGL((tq_input_kernel<SRC, BF16, 2>), dim3((unsigned)items), dim3(64), 0, st, src, (long long)K,
+                         (int)r0, (int)items, nout, p, scale);
+    else
+      hipLaunchKernelGGL((tq_input_kernel<SRC, BF16, 8>), dim3((unsigned)((items + 15) / 16)), dim3(256), 0, st, src,
+                         (long long)K, (int)r0, (int)items, nout, p, scale);
   }
 }
 
@@ -77,12 +95,9 @@ void input_run(bool bf16, int64_t x, int64_t M, int64_t K, int nout, const int64
   }
   // float(2^s / sqrt(128)), rounded once from double (trellis_ref.hpp:146-148)
   const float scale = (float)(__builtin_ldexp(1.0, prescale_log2) / __builtin_sqrt(128.0));
-  dim3 grid((unsigned)(K / 128), (unsigned)M), block(64);
   const R4XSrc src{(const unsigned short*)x, nullptr, (long long)K, 0};
-  if (bf16)
-    hipLaunchKernelGGL((tq_input_kernel<R4_SRC_X, true>), grid, block, 0, (hipStream_t)stream, src, K, nout, p, scale);
-  else
-    hipLaunchKernelGGL((tq_input_kernel<R4_SRC_X, false>), grid, block, 0, (hipStream_t)stream, src, K, nout, p, scale);
+  if (bf16) input_launch<R4_SRC_X, true>(src, M, K, nout, p, scale, (hipStream_t)stream);
+  else input_launch<R4_SRC_X, false>(src, M, K, nout, p, scale, (hipStream_t)stream);
   r4d::launch_ok(entry);
 }
 
@@ -103,8 +118,7 @@ void producer_run(const R4XSrc& src, int64_t rows, int64_t K, int64_t suh, int64
   OutPtrs p{};
   p.suh[0] = (const float*)suh;
   p.out[0] = (unsigned short*)out;
-  hipLaunchKernelGGL((tq_input_kernel<SRC, true>), dim3((unsigned)(K / 128), (unsigned)rows), dim3(64), 0,
-                     (hipStream_t)stream, src, K, 1, p, scale);
+  input_launch<SRC, true>(src, rows, K, 1, p, scale, (hipStream_t)stream);
   r4d::launch_ok(entry);
 }
 

@@ -473,91 +473,70 @@ __global__ __launch_bounds__(64 * kM2Waves, 1) void tq_m256_kernel(
 }
 #undef M2_SEGMENT_BEGIN
 
-// The split form's second pass: a workgroup per (128-column group, 16 rows) sums the SKG slices of ws in
-// slice order into LDS, then one wave per row applies the group's FWHT-128 (r4_fwht128_wave, the reference's
-// stage order), svh, out_scale and the bf16 rounding -- or, raw, stores the fp32 sums. Up to 8 slices (one per
-// run): a thread takes 4 adjacent columns of 2 rows and requests all 8 slices of them at once as 16-byte
-// loads (a slice past SKG reads past the buffer and returns 0, which is exactly what an empty run adds), so
-// one memory round trip covers the workgroup; more slices take the general loop (a thread per column).
-constexpr int kFinRows = 16;
+// The split form's second pass: 16 lanes per (row, 128-column group), 8 adjacent columns per lane, sum the SKG slices of
+// ws in the M <= 64 kernel's order (run p (0..7) = 0.f + slices p, p + 8, ... in order, then the runs in order 0..7; an
+// absent slice adds +0.f, which changes nothing), apply the FWHT-128 (r4_fwht128_rows), svh, out_scale and the bf16
+// rounding, and store 16 bytes -- or, raw, the fp32 sums. Memory-bound: every slice of a batch of 8 is requested (16-byte
+// loads) before any is added, and nothing passes through LDS (256 x 5120 in 4 slices 6.2 -> 5.4 us, 256 x 8192 in 4
+// 8.5 -> 7.3 us against a version that summed through LDS and stored two bytes per lane).
+constexpr int kFinRows = 16;   // rows of a workgroup
 __global__ __launch_bounds__(256) void tq_m256_finish(const float* __restrict__ ws, const float* __restrict__ svh,
                                                       void* __restrict__ Cv, int M, int N, int SKG, int full,
                                                       float out_scale) {
-  __shared__ float sums[kFinRows][128];
-  const int group = blockIdx.x, r0 = blockIdx.y * kFinRows;
-  const int n0 = group * 128;
+  const int lane = threadIdx.x & 63;
+  const int r = blockIdx.y * kFinRows + (threadIdx.x >> 4), col = blockIdx.x * 128 + 8 * (lane & 15);
   const size_t sy = (size_t)M * N;
-  // the M <= 64 kernel's slice order: run p (0..7) = 0.f + slices p, p + 8, ... in order, then the 8 runs
-  // added in order 0..7
-  if (SKG <= 8) {
-    const int cq = threadIdx.x & 31, rr = threadIdx.x >> 5;      // columns 4 cq .. 4 cq + 3, rows rr, rr + 8
-    const unsigned sy4 = (unsigned)sy * 4u;
-    const r4_rsrc wr = mk_rsrc(ws, (unsigned)SKG * sy4);
+  const float* src = ws + (size_t)r * N + col;
+  float sv[8];
+  if (full) r4_load_f32<8>(svh + col, sv);
+  float v[8];
+  if (SKG <= 8) {   // at most one slice per run (every planned split)
     r4f4 t[8][2];
 #pragma unroll
     for (int p = 0; p < 8; ++p)
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const unsigned off = (unsigned)p * sy4 + (unsigned)((r0 + rr + 8 * u) * N + n0 + 4 * cq) * 4u;
-        t[p][u] = __builtin_bit_cast(r4f4, __builtin_amdgcn_raw_buffer_load_b128(wr, off, 0, 0));
+      if (p < SKG) {
+        t[p][0] = *(const r4f4_a4*)(src + p * sy);
+        t[p][1] = *(const r4f4_a4*)(src + p * sy + 4);
       }
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      float v[4];
+    for (int e = 0; e < 8; ++e) v[e] = 0.f + t[0][e >> 2][e & 3];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float acc = 0.f + t[0][u][e];
+    for (int p = 1; p < 8; ++p)
+      if (p < SKG) {
 #pragma unroll
-        for (int p = 1; p < 8; ++p) acc = acc + (0.f + t[p][u][e]);
-        v[e] = acc;
+        for (int e = 0; e < 8; ++e) v[e] += 0.f + t[p][e >> 2][e & 3];
       }
-      const int r = rr + 8 * u;
-      if (!full) {
-        *(r4f4*)((float*)Cv + (size_t)(r0 + r) * N + n0 + 4 * cq) = (r4f4){v[0], v[1], v[2], v[3]};
-      } else {
+    if (SKG < 8) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sums[r][4 * cq + e] = v[e];
-      }
+      for (int e = 0; e < 8; ++e) v[e] += 0.f;
     }
-    if (!full) return;
   } else {
-    const int col = threadIdx.x & 127, rh = threadIdx.x >> 7;   // rows rh + 2 u
-    float v[kFinRows / 2];
 #pragma unroll 1
     for (int p = 0; p < 8; ++p) {
-      float run[kFinRows / 2];
-#pragma unroll
-      for (int u = 0; u < kFinRows / 2; ++u) run[u] = 0.f;
+      float run[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       for (int y = p; y < SKG; y += 8) {
-        float t[kFinRows / 2];
+        const r4f4 a = *(const r4f4_a4*)(src + y * sy), b = *(const r4f4_a4*)(src + y * sy + 4);
 #pragma unroll
-        for (int u = 0; u < kFinRows / 2; ++u) t[u] = ws[(size_t)y * sy + (size_t)(r0 + rh + 2 * u) * N + n0 + col];
-#pragma unroll
-        for (int u = 0; u < kFinRows / 2; ++u) run[u] += t[u];
+        for (int e = 0; e < 4; ++e) {
+          run[e] += a[e];
+          run[4 + e] += b[e];
+        }
       }
 #pragma unroll
-      for (int u = 0; u < kFinRows / 2; ++u) v[u] = p == 0 ? run[u] : v[u] + run[u];
+      for (int e = 0; e < 8; ++e) v[e] = p == 0 ? run[e] : v[e] + run[e];
     }
-    if (!full) {
-      float* Cf = (float*)Cv;
-#pragma unroll
-      for (int u = 0; u < kFinRows / 2; ++u) Cf[(size_t)(r0 + rh + 2 * u) * N + n0 + col] = v[u];
-      return;
-    }
-#pragma unroll
-    for (int u = 0; u < kFinRows / 2; ++u) sums[rh + 2 * u][col] = v[u];
   }
-  __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  unsigned short* Cb = (unsigned short*)Cv;
-  const float sv0 = svh[n0 + lane], sv1 = svh[n0 + lane + 64];
-  for (int r = wave; r < kFinRows; r += 4) {
-    float v0 = sums[r][lane], v1 = sums[r][lane + 64];
-    r4_fwht128_wave(v0, v1, lane);
-    const float y0 = v0 * sv0, y1 = v1 * sv1;
-    Cb[(size_t)(r0 + r) * N + n0 + lane] = r4_bf16_rn(y0 * out_scale);
-    Cb[(size_t)(r0 + r) * N + n0 + lane + 64] = r4_bf16_rn(y1 * out_scale);
+  if (!full) {
+    float* dst = (float*)Cv + (size_t)r * N + col;
+    *(r4f4_a4*)dst = (r4f4){v[0], v[1], v[2], v[3]};
+    *(r4f4_a4*)(dst + 4) = (r4f4){v[4], v[5], v[6], v[7]};
+    return;
   }
+  r4_fwht128_rows<8>(v, lane);
+  unsigned h[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) h[e] = r4_bf16_rn_sel((v[e] * sv[e]) * out_scale);
+  r4_store_u16<8>((unsigned short*)Cv + (size_t)r * N + col, h);
 }
 
 std::string m256_check(int M, int K, int N, int n_split, int KB, int SKG) {
