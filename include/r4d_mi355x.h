@@ -30,7 +30,8 @@ extern "C" {
 /* third_party/libr4d/r4d.h:372-375 r4d_gemm_trellis_nt_m64: C bf16 [M][N] =
  * bf16((FWHT128(A_p(n) @ Q) * svh) * out_scale); A f16 [M][K] (a1 = 0: a0), W the pair-grid words,
  * ws fp32 ws_bytes(M, N, SKG) (SKG M N 4 at most 2 GiB), tickets tickets_bytes(N) (one 128-byte line per
- * 128-column group) zeroed before first use (self-resetting). */
+ * 128-column group) zeroed before first use (self-resetting). Above 16 rows an unsplit launch (SKG = 1) in the SK 1 / 2
+ * order uses both where they are given: units cut between workgroups are handed on through them, the bits unchanged. */
 void r4d_gemm_trellis_nt_m64(int64_t a0, int64_t a1, int n_split, int64_t w, int64_t svh, int64_t c,
                              int64_t ws, int64_t tickets, int M, int K, int N, int KB, int WV, int SK,
                              int MT, int NP, int SKG, int U, int NT, float out_scale, int64_t stream);

@@ -35,6 +35,8 @@ MIN_OCCUPANCY = [            # (demangled name prefix, waves per SIMD at least):
     ("tq_gemv_kernel<4, 1, 2, 4, true, 0, false>", 6),   # ... at M = 2..16
     ("tq_gemv_kernel<5, 1, 1, 4, true, 0, false>", 5),
     ("tq_gemv_kernel<", 2),
+    ("tq_mid_kernel<", 1),       # 17..64 rows; the fake-quant forms take what they need
+    ("tq_mid_kernel<4, 2, 1, false>", 2), ("tq_mid_kernel<4, 2, 4, false>", 4), ("tq_mid_kernel<4, 4, 4, false>", 4),
     ("tq_m256_kernel<", 2),      # 8 waves of 64, one workgroup per CU (96 KiB of LDS stages)
     ("tq_m256_finish", 4),
     ("ti8_gemm_kernel<", 2),     # 8 waves, one workgroup per CU
@@ -42,9 +44,9 @@ MIN_OCCUPANCY = [            # (demangled name prefix, waves per SIMD at least):
     ("am_kernel<", 8),
 ]
 # Kernels allowed a few SGPR spills (at most this many; they go to VGPR lanes by v_writelane, never to memory, and the
-# gate still requires no scratch and no VGPR spill): the prefill GEMM keeps its launch arguments and the per-segment
-# geometry of the balanced form in scalars across the whole kernel, outside the step loop.
-SGPR_LANE_SPILLS = [("tq_m256_kernel<", 16)]
+# gate still requires no scratch and no VGPR spill): the prefill GEMM and the 17..64-row kernel keep their launch arguments
+# and the per-segment geometry of the balanced form in scalars across the whole kernel, outside the step loop.
+SGPR_LANE_SPILLS = [("tq_m256_kernel<", 16), ("tq_mid_kernel<", 48)]
 
 
 def parse_resources(text):

@@ -4,6 +4,8 @@
 #pragma once
 #include "r4d_dev.h"
 
+#include <type_traits>
+
 namespace {
 
 template <int KB>
@@ -113,7 +115,8 @@ struct TqOut {
 // LDS bytes of a unit's end: the part accumulators (dead before the group's sums are formed in the same bytes), then
 // the ticket flag.
 constexpr size_t tq_end_lds_flag(int MT, int NPW, int SK, int M) {
-  const size_t parts = (size_t)(SK - 1) * NPW * 8 * MT * 64 * 4, sums = NPW == 4 ? (size_t)M * 128 * 4 : 0;
+  const size_t parts = (size_t)(SK - 1) * NPW * 8 * MT * 64 * 4;
+  const size_t sums = MT > 1 || NPW == 4 ? (size_t)M * NPW * 32 * 4 : 0;
   return parts > sums ? parts : sums;
 }
 constexpr size_t tq_end_lds(int MT, int NPW, int SK, int M) { return tq_end_lds_flag(MT, NPW, SK, M) + 16; }
@@ -122,7 +125,8 @@ constexpr size_t tq_end_lds(int MT, int NPW, int SK, int M) { return tq_end_lds_
 // of fragment cs: true column 32 pair + 16 (nb >> 3) + (nb & 7) + 8 cs.
 //   * SKG = 1, raw: the sums are C.
 //   * SKG = 1 in a workgroup that holds its whole group (NPW = 4): the sums meet in LDS.
-//   * else the partials go to ws and the last of the group's SKG 4 / NPW contributors (ticket) sums the slices: run p
+//   * else the partials go to ws -- above one row tile through LDS, as 16-byte row pieces (the accumulators' own 4-byte
+//     stores cost 3 to 5 us a launch at 49 and 64 rows) -- and the last of the group's SKG 4 / NPW contributors (ticket) sums the slices: run p
 //     (0..7) is 0.f + slices p, p + 8, ... in order, then the runs in order 0..7 (an absent slice adds +0.f, which changes
 //     nothing) -- the same arithmetic for every element whatever M is. The loads are coherent (sc1) 16-byte buffer loads,
 //     every slice of a batch of 8 requested before any is added.
@@ -156,20 +160,36 @@ __device__ __forceinline__ void tq_finish(const r4f4 (&acc)[MT][2], unsigned cha
     return;
   }
   const bool in_block = NPW == 4 && SK == 1 && SKG == 1;   // the workgroup holds its whole group
-  if (in_block) {
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int r = 16 * i + 4 * rq + j;
-        if (r < M) {
-          red[r * 128 + gcol0] = acc[i][0][j];
-          red[r * 128 + gcol0 + 8] = acc[i][1][j];
-        }
-      }
-    __syncthreads();
-  } else {
+  constexpr bool kStaged = MT > 1;              // the partials pass through LDS and leave as whole 16-byte row pieces
+  constexpr int kCols = 32 * NPW;               // the workgroup's columns
+  const unsigned sy4 = (unsigned)M * (unsigned)N * 4u;
+  const r4_rsrc wsr = r4_make_rsrc(o.ws, (unsigned)SKG * sy4);
+  if (in_block || kStaged) {
+    if constexpr (SK > 1) __syncthreads();      // the part accumulators have been read
+    const int lcol0 = gcol0 & (kCols - 1);
     if (ks == 0) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int r = 16 * i + 4 * rq + j;
+          if (r < M) {
+            red[r * kCols + lcol0] = acc[i][0][j];
+            red[r * kCols + lcol0 + 8] = acc[i][1][j];
+          }
+        }
+    }
+    __syncthreads();
+  }
+  if (!in_block) {
+    if constexpr (kStaged) {
+      const unsigned base = (unsigned)ky * sy4 + (unsigned)(n0 + (kCols == 128 ? 0 : (pair * 32) & (128 - kCols))) * 4u;
+      for (int it = (int)threadIdx.x; it < M * (kCols / 4); it += NT) {
+        const int r = it / (kCols / 4), cq = it & (kCols / 4 - 1);
+        __builtin_amdgcn_raw_buffer_store_b128(*(const r4u4*)(red + r * kCols + 4 * cq), wsr,
+                                               base + (unsigned)r * (unsigned)N * 4u + 16u * cq, 0, 16);
+      }
+    } else if (ks == 0) {
       float* wsy = o.ws + (size_t)ky * M * N;
 #pragma unroll
       for (int i = 0; i < MT; ++i)
@@ -186,63 +206,84 @@ __device__ __forceinline__ void tq_finish(const r4f4 (&acc)[MT][2], unsigned cha
                         (int*)(lds + tq_end_lds_flag(MT, NPW, SK, M))))
       return;
   }
-  const unsigned sy4 = (unsigned)M * (unsigned)N * 4u;
-  const r4_rsrc wsr = r4_make_rsrc(o.ws, (unsigned)SKG * sy4);
   const int c0 = 4 * (lane & 31);               // this lane's 4 columns
-  for (int it = (int)threadIdx.x; it < M * 32; it += NT) {
-    const int r = it >> 5;
-    float v[4], sv[4];
-    if (full) r4_load_f32<4>(o.svh + n0 + c0, sv);   // requested with the slices
+  float sv[4] = {0.f, 0.f, 0.f, 0.f};
+  if (full) r4_load_f32<4>(o.svh + n0 + c0, sv);
+  // rows per thread and pass, all their slices requested at once (one row at a time, a workgroup at 49 rows made seven
+  // memory round trips one after the other)
+  constexpr int kU = MT == 1 || (MT == 4 && SK == 4) ? 1 : 2;
+  for (int it0 = (int)threadIdx.x; it0 < M * 32; it0 += kU * NT) {
+    float v[kU][4];
     if (in_block) {
-      const r4f4 a = *(const r4f4*)(red + r * 128 + c0);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = a[e];
+      for (int u = 0; u < kU; ++u) {
+        const r4f4 a = *(const r4f4*)(red + min((it0 + u * NT) >> 5, M - 1) * kCols + (c0 & (kCols - 1)));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[u][e] = a[e];
+      }
     } else {
-      const unsigned off = ((unsigned)r * (unsigned)N + (unsigned)(n0 + c0)) * 4u;
-      auto slice = [&](int y) {
-        return __builtin_bit_cast(r4f4, __builtin_amdgcn_raw_buffer_load_b128(wsr, off + (unsigned)y * sy4, 0, 16));
+      unsigned off[kU];
+#pragma unroll
+      for (int u = 0; u < kU; ++u)
+        off[u] = ((unsigned)min((it0 + u * NT) >> 5, M - 1) * (unsigned)N + (unsigned)(n0 + c0)) * 4u;
+      auto slice = [&](int u, unsigned sy) {
+        return __builtin_bit_cast(r4f4, __builtin_amdgcn_raw_buffer_load_b128(wsr, off[u] + sy, 0, 16));
       };
-      if (SKG <= 8) {   // at most one slice per run (every planned split)
-        r4f4 t[8];
+      // at most one slice per run (every planned split): branch-free, a slice past SKG reads past the buffer and gives the
+      // +0.f of an empty run (a load under a branch would also keep its registers live around the caller's loop)
+      auto few = [&](auto n) {
+        constexpr int kN = decltype(n)::value;
+        r4f4 t[kU][kN];
 #pragma unroll
-        for (int p = 0; p < 8; ++p)
-          if (p < SKG) t[p] = slice(p);
+        for (int u = 0; u < kU; ++u)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = 0.f + t[0][e];
+          for (int p = 0; p < kN; ++p) t[u][p] = slice(u, p < SKG ? (unsigned)p * sy4 : 0x80000000u);
 #pragma unroll
-        for (int p = 1; p < 8; ++p)
-          if (p < SKG) {
+        for (int u = 0; u < kU; ++u)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] += 0.f + t[p][e];
+          for (int e = 0; e < 4; ++e) {
+            v[u][e] = 0.f + t[u][0][e];
+#pragma unroll
+            for (int p = 1; p < kN; ++p) v[u][e] += 0.f + t[u][p][e];
+            if (kN < 8) v[u][e] += 0.f;
           }
-        if (SKG < 8) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] += 0.f;
-        }
+      };
+      if (SKG <= 4) {
+        few(std::integral_constant<int, 4>());
+      } else if (SKG <= 8) {
+        few(std::integral_constant<int, 8>());
       } else {
-#pragma unroll 1
-        for (int p = 0; p < 8; ++p) {
-          float run[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-          for (int y = p; y < SKG; y += 8) {
-            const r4f4 t = slice(y);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) run[e] += t[e];
+        for (int u = 0; u < kU; ++u) {
+#pragma unroll 1
+          for (int p = 0; p < 8; ++p) {
+            float run[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+            for (int y = p; y < SKG; y += 8) {
+              const r4f4 t = slice(u, (unsigned)y * sy4);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) run[e] += t[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[u][e] = p == 0 ? run[e] : v[u][e] + run[e];
           }
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = p == 0 ? run[e] : v[e] + run[e];
         }
       }
     }
-    if (!full) {
-      *(r4f4_a4*)(Cf + (size_t)r * N + n0 + c0) = (r4f4){v[0], v[1], v[2], v[3]};
-      continue;
-    }
-    r4_fwht128_rows<4>(v, lane);
-    unsigned h[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) h[e] = r4_bf16_rn_sel((v[e] * sv[e]) * o.out_scale);
-    r4_store_u16<4>(Cb + (size_t)r * N + n0 + c0, h);
+    for (int u = 0; u < kU; ++u) {
+      const int it = it0 + u * NT, r = it >> 5;
+      if (full) r4_fwht128_rows<4>(v[u], lane);
+      if (it >= M * 32) break;
+      if (!full) {
+        *(r4f4_a4*)(Cf + (size_t)r * N + n0 + c0) = (r4f4){v[u][0], v[u][1], v[u][2], v[u][3]};
+        continue;
+      }
+      unsigned h[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) h[e] = r4_bf16_rn_sel((v[u][e] * sv[e]) * o.out_scale);
+      r4_store_u16<4>(Cb + (size_t)r * N + n0 + c0, h);
+    }
   }
 }
 

@@ -1,5 +1,5 @@
-// trellis_gemv.hip -- the trellis linear for M = 1..64 rows on gfx950: r4d_gemm_trellis_nt_m64, its
-// _raw fp32 entry, r4d_trellis_reconstruct_f16 and the ticket helpers (the C ABI of the reference's
+// trellis_gemv.hip -- the trellis linear for M = 1..64 rows on gfx950 (the kernel of M <= 16 and of the fused input
+// transform; trellis_mid.hip has 17..64): r4d_gemm_trellis_nt_m64, its _raw fp32 entry, r4d_trellis_reconstruct_f16 and the ticket helpers (the C ABI of the reference's
 // third_party/libr4d/r4d.h:344-393, kernel semantics of r4d_gemm_trellis_nt_m64.hip:215-503).
 //
 // C[m][n] = bf16((FWHT128(A_p(n) @ Q)[m][n] * svh[n]) * out_scale)   (full), or fp32 A @ Q (_raw).
@@ -57,9 +57,7 @@ __global__ __launch_bounds__(64 * NPW * SK, MT == 1 && ALDS && SK == 4 && XF == 
     float* __restrict__ ws, unsigned* __restrict__ tickets, int M, int K, int N, int SKG, int full,
     float out_scale, const R4SParts sp, float xscale,
     unsigned long long* __restrict__ clk, const float* __restrict__ wsc, int wq_gsh) {
-  // steps in flight; 2 where each ring slot also carries MT row tiles of A from global memory (4 slots of 4 row
-  // tiles would not fit the VGPRs and spill)
-  constexpr int PF = (!ALDS && MT >= 4) ? 2 : 4;
+  constexpr int PF = 4;                        // steps in flight
   constexpr int NT = 64 * NPW * SK;
   constexpr int NW = NPW * SK;                 // waves
   constexpr int BLK = 16 * KB;                 // words per (pair, k-tile) block
@@ -480,17 +478,19 @@ void launch_gemv_a(const r4d_gemv_args& a) {
     if (abytes > kXfAldsMax) r4d::fail("trellis_gemv_xf", "the A slice does not fit LDS: raise SKG");
     if (a.xf == 2) launch_gemv<KB, MT, NPW, SK, true, 2>(a);
     else launch_gemv<KB, MT, NPW, SK, true, 1>(a);
-  } else if (a.wsc) {
-    if constexpr (KB == 4 || KB == 5) {
-      if (abytes <= kAldsMax) launch_gemv<KB, MT, NPW, SK, true, 0, true>(a);
-      else launch_gemv<KB, MT, NPW, SK, false, 0, true>(a);
+  } else if constexpr (MT == 1) {
+    if (a.wsc) {
+      if constexpr (KB == 4 || KB == 5) {
+        if (abytes <= kAldsMax) launch_gemv<KB, MT, NPW, SK, true, 0, true>(a);
+        else launch_gemv<KB, MT, NPW, SK, false, 0, true>(a);
+      } else {
+        r4d::fail("gemm_trellis_nt_m64_wq", "KB must be 4 or 5");
+      }
+    } else if (abytes <= kAldsMax) {
+      launch_gemv<KB, MT, NPW, SK, true, 0>(a);
     } else {
-      r4d::fail("gemm_trellis_nt_m64_wq", "KB must be 4 or 5");
+      launch_gemv<KB, MT, NPW, SK, false, 0>(a);
     }
-  } else if (abytes <= kAldsMax) {
-    launch_gemv<KB, MT, NPW, SK, true, 0>(a);
-  } else {
-    launch_gemv<KB, MT, NPW, SK, false, 0>(a);
   }
 }
 
@@ -499,19 +499,20 @@ void launch_gemv_a(const r4d_gemv_args& a) {
 // M >= 2 (measured best; the pairs of a workgroup are independent, so the form does not change a bit,
 // and fewer workgroups take fewer tickets on the group's counter).
 template <int KB, int MT>
-void launch_gemv_np(const r4d_gemv_args& a) {
-  const GemvForm f = gemv_form(a.M, a.N, a.SKG, a.ws != 0 && a.tickets != 0, a.sk1 != 0, a.xf != 0);
+void launch_gemv_np(const r4d_gemv_args& a, const GemvForm& f) {
   if (f.SK == 1) launch_gemv_a<KB, MT, 4, 1>(a);
   else if (f.NPW == 1) launch_gemv_a<KB, MT, 1, 4>(a);
   else launch_gemv_a<KB, MT, 2, 4>(a);
 }
 
+// More than one row tile runs here only with the fused transform (A staged whole); trellis_mid.hip has the other forms.
 template <int KB>
-void launch_gemv_kb(const r4d_gemv_args& a) {
-  const int mt = gemv_form(a.M, a.N, a.SKG, true, false).MT;
-  if (mt <= 1) launch_gemv_np<KB, 1>(a);
-  else if (mt <= 2) launch_gemv_np<KB, 2>(a);
-  else launch_gemv_np<KB, 4>(a);
+void launch_gemv_kb(const r4d_gemv_args& a, const char* entry) {
+  const GemvForm f = gemv_form(a.M, a.N, a.SKG, a.ws != 0 && a.tickets != 0, a.sk1 != 0, a.xf != 0);
+  if (f.MT > 1 && !a.xf) r4d::gemv_mid(a, f.SK == 1, entry);
+  else if (f.MT <= 1) launch_gemv_np<KB, 1>(a, f);
+  else if (f.MT <= 2) launch_gemv_np<KB, 2>(a, f);
+  else launch_gemv_np<KB, 4>(a, f);
 }
 
 }  // namespace
@@ -522,9 +523,9 @@ void r4d::gemv_run(r4d_gemv_args& a, const char* entry) {
   if (const char* m = r4d_gemm_trellis_nt_m64_check(a.M, a.K, a.N, a.n_split, a.KB, a.SKG, a.full,
                                                     a.svh != 0, a.ws != 0 && a.tickets != 0))
     r4d::fail(entry, m);
-  if (a.KB == 4) launch_gemv_kb<4>(a);
-  else if (a.KB == 5) launch_gemv_kb<5>(a);
-  else launch_gemv_kb<3>(a);
+  if (a.KB == 4) launch_gemv_kb<4>(a, entry);
+  else if (a.KB == 5) launch_gemv_kb<5>(a, entry);
+  else launch_gemv_kb<3>(a, entry);
   r4d::launch_ok(entry);
 }
 
@@ -690,9 +691,9 @@ void r4dx_trellis_gemv_xf(int64_t x, int x_is_bf16, int64_t suh0, int64_t suh1, 
   a.xf = x_is_bf16 ? 2 : 1;
   // float(2^s / sqrt(128)), rounded once from double (trellis_ref.hpp:146-148)
   a.xscale = (float)(__builtin_ldexp(1.0, prescale_log2) / __builtin_sqrt(128.0));
-  if (a.KB == 4) launch_gemv_kb<4>(a);
-  else if (a.KB == 5) launch_gemv_kb<5>(a);
-  else launch_gemv_kb<3>(a);
+  if (a.KB == 4) launch_gemv_kb<4>(a, entry);
+  else if (a.KB == 5) launch_gemv_kb<5>(a, entry);
+  else launch_gemv_kb<3>(a, entry);
   r4d::launch_ok(entry);
 }
 
@@ -728,9 +729,9 @@ void r4dx_trellis_gemv_xf_parts(int64_t x, int x_is_bf16, const int64_t* suh, co
   a.suh3 = parts > 3 ? suh[3] : 0;
   a.xf = x_is_bf16 ? 2 : 1;
   a.xscale = (float)(__builtin_ldexp(1.0, prescale_log2) / __builtin_sqrt(128.0));
-  if (a.KB == 4) launch_gemv_kb<4>(a);
-  else if (a.KB == 5) launch_gemv_kb<5>(a);
-  else launch_gemv_kb<3>(a);
+  if (a.KB == 4) launch_gemv_kb<4>(a, entry);
+  else if (a.KB == 5) launch_gemv_kb<5>(a, entry);
+  else launch_gemv_kb<3>(a, entry);
   r4d::launch_ok(entry);
 }
 

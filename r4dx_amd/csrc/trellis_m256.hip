@@ -12,8 +12,8 @@
 // are M x N fp32 per slice) writes each slice to ws and a second launch, tq_m256_finish, adds the slices in order
 // and finishes. Unit counts that are not a multiple of the compute units run in the balanced form (one workgroup per
 // CU over an even share of the steps, a cut unit's accumulators handed on exactly; see the kernel).
-#include "r4d_dev.h"
 #include "r4d_host.h"
+#include "tq_units.h"
 #include "r4d_mi355x.h"
 
 namespace {
@@ -46,56 +46,6 @@ __device__ __forceinline__ int m2_slot(int r, int c) { return (r * 8 + (c ^ m2_s
 // flipped on odd 16-column tiles to keep the t = 0 and t = 1 lanes of one write on different banks; a
 // fragment read (16 consecutive columns of one chunk) stays a permutation of 16 bank slots.
 __device__ __forceinline__ int m2_bslot(int n, int c) { return c * 2048 + ((n ^ (((n >> 4) & 1) << 3)) * 16); }
-
-// The work of a launch is U = (N / 128) * SKG units -- unit u = group * SKG + y is K slice y of column group u / SKG
-// -- of nst steps each, taken in unit order. Data-parallel (P = 0): workgroup (group, y) takes one unit. Balanced
-// (P > 0 workgroups, used when U exceeds the CUs and is not a multiple of them): workgroup c takes the steps
-// an even share (T / P, one more for the first T % P) of the T = U nst, P <= U so that a range spans at most the end of one unit, whole units
-// and the start of one more. A unit cut by a range boundary stays one fold from 0.f in k order: the workgroup that
-// holds its start runs that part FIRST and publishes the fp32 accumulators (fix[c], M x 128; then flags[4 c] = 1),
-// the workgroup that holds the rest runs it LAST, starting from those accumulators (so every element is the same
-// sum, bit for bit). Workgroups are dispatched in index order and the publisher's part is its first work, so the
-// wait cannot deadlock; it is bounded anyway, and a wait that runs out poisons its results with NaN.
-constexpr int kSegWhole = 0, kSegPublish = 1, kSegContinue = 2;
-constexpr int kFlagStride = 4;            // words between two workgroups' flags
-// Workgroup c's flag is word kFlagStride c + 1 of the ticket buffer: never word 32 g, the counter of 128-column group g
-// that the M <= 64 kernel's split hand-over takes tickets on, so a flag left set can never be read as a ticket count.
-__device__ __forceinline__ unsigned* m2_flag(unsigned* flags, unsigned c) { return flags + (size_t)c * kFlagStride + 1; }
-
-// A workgroup's share: steps [beg, end) of the launch's units in order (unit u = group * SKG + y, nst steps each).
-struct M2Share {
-  int ub, sb, ue, se, whole0, nseg;
-};
-__device__ __forceinline__ M2Share m2_share(int N, int SKG, int nst, int P) {
-  // T = (N / 128) * SKG * nst <= (N / 128) * K / 64 steps fits 32 bits; workgroup c gets T / P steps, one more for the
-  // first T % P workgroups
-  int beg, end;
-  if (P > 0) {
-    const unsigned T = (unsigned)(N / 128) * (unsigned)SKG * (unsigned)nst, q = T / (unsigned)P, r = T % (unsigned)P;
-    const unsigned c = blockIdx.x;
-    beg = (int)(c * q + (c < r ? c : r));
-    end = beg + (int)q + (c < r ? 1 : 0);
-  } else {
-    beg = (blockIdx.x * SKG + blockIdx.y) * nst;
-    end = beg + nst;
-  }
-  M2Share sh;
-  sh.ub = beg / nst; sh.sb = beg - sh.ub * nst; sh.ue = end / nst; sh.se = end - sh.ue * nst;
-  sh.whole0 = sh.sb ? sh.ub + 1 : sh.ub;
-  sh.nseg = (sh.se ? 1 : 0) + (sh.ue - sh.whole0) + (sh.sb ? 1 : 0);
-  return sh;
-}
-// Segment si in run order: the start of unit ue (published), the whole units, the rest of unit ub (continued).
-struct M2Seg {
-  int u, s0, s1, kind;
-};
-__device__ __forceinline__ M2Seg m2_seg(const M2Share& sh, int si, int nst) {
-  M2Seg g;
-  if (sh.se && si == 0) { g.u = sh.ue; g.s0 = 0; g.s1 = sh.se; g.kind = kSegPublish; }
-  else if (sh.sb && si == sh.nseg - 1) { g.u = sh.ub; g.s0 = sh.sb; g.s1 = nst; g.kind = kSegContinue; }
-  else { g.u = sh.whole0 + si - (sh.se ? 1 : 0); g.s0 = 0; g.s1 = nst; g.kind = kSegWhole; }
-  return g;
-}
 
 // SK4: the M <= 64 kernel's 4-wave order (its SK 4, 8 and 16): each K slice's steps are cut into 4 contiguous parts of
 // ceil(steps / 4) steps, each part summed from 0.f, the parts added in order ((p0 + p1) + p2) + p3 (an empty part adds
@@ -552,27 +502,6 @@ std::string m256_check(int M, int K, int N, int n_split, int KB, int SKG) {
   return "";
 }
 
-// The device's compute units (cached per device).
-int m256_cus() {
-  static int cache[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cache[dev] == 0) {
-    int n = 0;
-    cache[dev] = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
-  }
-  return cache[dev];
-}
-// Workgroups of the balanced form for a launch of U units (0: data-parallel): used when U exceeds the compute units and
-// is not a multiple of them, and ws (for the published accumulators) and the tickets (for the flags) are there.
-int m256_balanced_p(int M, int N, int SKG, bool have_ws, bool have_tickets) {
-  (void)M;
-  const int G = N / 128, U = G * SKG, cus = m256_cus();
-  if (!have_ws || !have_tickets || U <= cus || U % cus == 0) return 0;
-  if ((long long)cus * kFlagStride + 1 > (long long)G * R4_TICKET_WORDS) return 0;   // the flags fit the ticket buffer
-  return cus;
-}
-
 template <int KB, int RT, bool WQ, bool SK4 = false>
 void m256_launch_rt(const R4AParts& ap, const unsigned* w,
                     const float* svh, void* c, float* ws, unsigned* tickets, int M, int K, int N, int SKG, int full,
@@ -580,7 +509,7 @@ void m256_launch_rt(const R4AParts& ap, const unsigned* w,
   constexpr unsigned lds = 2 * (32 * RT * 128 + 128 * 128);
   static std::atomic<unsigned long long> lds_set{0};
   r4d::allow_lds((const void*)tq_m256_kernel<KB, RT, WQ, SK4>, lds_set, "gemm_trellis_nt_m256");
-  const int P = SK4 ? 0 : m256_balanced_p(M, N, SKG, ws != nullptr, tickets != nullptr);
+  const int P = SK4 ? 0 : r4_balanced_p(N, SKG, ws != nullptr, tickets != nullptr);
   // the published accumulators follow the SKG slices in ws (SKG = 1: no slices, they start at ws)
   float* fix = ws ? ws + (SKG > 1 ? (size_t)SKG * M * N : 0) : nullptr;
   const dim3 grid = P > 0 ? dim3(P) : dim3(N / 128, SKG);
@@ -701,7 +630,7 @@ size_t r4d_gemm_trellis_nt_m256_ws_bytes(int M, int N, int SKG) {
   if (M <= 0 || N <= 0 || SKG <= 0) return 0;
   const size_t slices = (size_t)SKG * (size_t)M * (size_t)N * sizeof(float);
   if (SKG == 1) return slices;
-  const size_t units = (size_t)(N / 128) * (size_t)SKG, cus = (size_t)m256_cus();
+  const size_t units = (size_t)(N / 128) * (size_t)SKG, cus = (size_t)r4_cus();
   return slices + (units < cus ? units : cus) * (size_t)M * 128 * sizeof(float);
 }
 
@@ -758,7 +687,7 @@ int r4d_mi355x_trellis_m256_skg(int K, int N, int KB) {
   (void)KB;
   const int KT = K / 16, G = N / 128;
   if (KT <= 0 || G <= 0) return 1;
-  const int cus = m256_cus();
+  const int cus = r4_cus();
   int best = 1;
   double best_cost = 1e30;
   for (int d = 1; d <= 8; d *= 2) {
