@@ -213,6 +213,10 @@ void r4d_gemm_trellis_nt_i8(int64_t a8_0, int64_t sa_0, int64_t a8_1, int64_t sa
                             int KB, int skw, int skg, float out_scale, int64_t stream);
 const char* r4d_gemm_trellis_nt_i8_check(int M, int K, int N, int n_split, int KB, int skw, int skg);
 size_t r4d_gemm_trellis_nt_i8_ws_bytes(int M, int N, int SKG);
+/* No reference counterpart (the reference reads gemm_tuning_table_trellis_i8*.inc): this build's skg of the two trellis
+ * int8 GEMMs for a shape. With skg > 1 and more column groups than compute units, not a multiple of them, only the groups
+ * beyond the last whole round are cut along K (in up to 8 pieces, whatever skg is; the others are summed whole). */
+int    r4d_mi355x_trellis_i8_skg(int K, int N);
 /* r4d.h:514-521: the coarse sibling: SWC [N] (one scale per column over K), SA [256] (per row, from
  * r4d_trellis_i8_quant_act_row), the int32 sum of the slice scaled once by sa[row] * swc[col]. */
 size_t r4d_trellis_i8_wscale_col_count(int K, int N);

@@ -22,8 +22,8 @@
 // 16 bytes an MFMA lane needs in A8's k order, so nothing is permuted. Unsplit, the FWHT-128 epilogue runs
 // in registers (column bits 0-3 across lanes, 4-6 across column tiles); split K writes fp32 slices to ws
 // and the split finish pass (trellis_m256.hip) adds them in order and runs the same epilogue.
-#include "r4d_dev.h"
 #include "r4d_host.h"
+#include "tq_units.h"
 #include "r4d_mi355x.h"
 
 namespace {
@@ -188,6 +188,9 @@ struct TI8Args {
   // arrive (ticket) adds all of them in piece order, then finishes the group
   int G, U;
   unsigned* tickets;
+  // tail split (tail_s > 1, trellis launches with SKG > 1): column groups below tail_f run whole, the others are cut into
+  // tail_s pieces of whole 128-k blocks whose sums go to ws [piece][256][128 (N / 128 - tail_f)]
+  int tail_f, tail_s;
 };
 constexpr int kStreamG = 256;                   // workgroups of a stream-K launch (one per CU)
 constexpr int kSlot = 256 * 128;                // values per partial piece
@@ -202,10 +205,11 @@ __device__ __forceinline__ int ti8_unit_owner(int x, int U, int G) {
 }
 
 // One piece: column group `group`, k-tiles kt0 .. kt0 + 4 nst of it. slot < 0: the whole group's K range
-// (or a classic split slice ky); slot >= 0: a stream-K partial piece (see TI8Args).
+// (or a classic split slice ky); slot >= 0: a stream-K partial piece (see TI8Args). ws holds the columns from ws_n0 on;
+// whole: the group is finished here although SKG > 1.
 template <int KB, int SC, int OUT, bool DENSE>
 __device__ __forceinline__ void ti8_piece(const TI8Args& p, unsigned char (*bst)[4][128][16], int* flag, int group,
-                                          int ky, int kt0, int nst, int slot) {
+                                          int ky, int kt0, int nst, int slot, int ws_n0 = 0, bool whole = false) {
   constexpr bool BLKA = SC != kSCoarse;           // per-128 activation scales: fp32 accumulators
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -473,14 +477,15 @@ __device__ __forceinline__ void ti8_piece(const TI8Args& p, unsigned char (*bst)
           else v[ii][ct][j] = facc[ii][ct][j];
         }
     }
-    if (p.SKG > 1) {
-      float* dst = p.ws + (size_t)ky * 256 * N;
+    if (p.SKG > 1 && !whole) {
+      const int nw = N - ws_n0;
+      float* dst = p.ws + (size_t)ky * 256 * nw + (n0 - ws_n0);
 #pragma unroll
       for (int ii = 0; ii < 2; ++ii)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int ct = 0; ct < 8; ++ct) dst[(size_t)(32 * wave + 16 * ii + 4 * g + j) * N + n0 + 16 * ct + r16] = v[ii][ct][j];
+          for (int ct = 0; ct < 8; ++ct) dst[(size_t)(32 * wave + 16 * ii + 4 * g + j) * nw + 16 * ct + r16] = v[ii][ct][j];
       return;
     }
     if constexpr (OUT == kOutF16) {
@@ -538,6 +543,20 @@ template <int KB, int SC, int OUT, bool DENSE>
 __global__ __launch_bounds__(512, 1) void ti8_gemm_kernel(TI8Args p) {
   __shared__ __attribute__((aligned(16))) unsigned char bst[2][4][128][16];   // [stage][k-tile][column slot][16 B]
   __shared__ int flag;
+  if constexpr (!DENSE) {
+    if (p.tail_s > 1) {
+      // the pieces first: a CU that ran one takes a whole group next, and the last round is whole groups only
+      const int pieces = (p.N / 128 - p.tail_f) * p.tail_s, b = blockIdx.x;
+      if (b < pieces) {
+        const int g = b / p.tail_s, y = b - g * p.tail_s, nb = p.K >> 7;
+        const int b0 = (int)((long long)y * nb / p.tail_s), b1 = (int)((long long)(y + 1) * nb / p.tail_s);
+        ti8_piece<KB, SC, OUT, DENSE>(p, bst, &flag, p.tail_f + g, y, 8 * b0, 2 * (b1 - b0), -1, 128 * p.tail_f);
+      } else {
+        ti8_piece<KB, SC, OUT, DENSE>(p, bst, &flag, b - pieces, 0, 0, p.K >> 6, -1, 0, true);
+      }
+      return;
+    }
+  }
   if (!DENSE || p.G == 0) {
     const int ktw = (p.K >> 4) / p.SKG;
     ti8_piece<KB, SC, OUT, DENSE>(p, bst, &flag, blockIdx.x, blockIdx.y, blockIdx.y * ktw, ktw >> 2, -1);
@@ -590,9 +609,32 @@ std::string ti8_check(int M, int K, int N, int n_split, int KB, int skw, int skg
   return "";
 }
 
+// The launch form of more column groups than compute units. Their groups in whole rounds run unsplit and only the
+// remainder's are cut along K, into as many pieces as fit one short round (at most 8, the split finish's fast form), so the
+// last round is short and only the remainder's sums pass through memory (256 x 128 fp32 per piece; they fit any split's
+// ws: pieces <= groups). s = 1: no remainder, or one too large to gain -- the K split as asked. 5120 x 34816 (272 groups
+// on 256 CUs), coarse / per-128: unsplit 131 / 180 us (two rounds), SKG 2 115 / 152, this 93 / 114.
+struct TI8Tail {
+  int f, s;
+};
+TI8Tail ti8_tail(int K, int N, int cus) {
+  const int G = N / 128, nb = K / 128, r = G % cus;
+  TI8Tail t{G, 1};
+  if (G <= cus || r == 0) return t;
+  int s = cus / r;
+  if (s > 8) s = 8;
+  if (s > nb) s = nb;
+  if (s < 2) return t;
+  t.f = G - r;
+  t.s = s;
+  return t;
+}
+
 template <int KB, int SC, int OUT, bool DENSE>
 void ti8_launch(const TI8Args& a, int N, int SKG, hipStream_t st) {
   if (a.G > 0) hipLaunchKernelGGL((ti8_gemm_kernel<KB, SC, OUT, DENSE>), dim3(a.G), dim3(512), 0, st, a);
+  else if (a.tail_s > 1)
+    hipLaunchKernelGGL((ti8_gemm_kernel<KB, SC, OUT, DENSE>), dim3(a.tail_f + (N / 128 - a.tail_f) * a.tail_s), dim3(512), 0, st, a);
   else hipLaunchKernelGGL((ti8_gemm_kernel<KB, SC, OUT, DENSE>), dim3(N / 128, SKG), dim3(512), 0, st, a);
 }
 
@@ -620,6 +662,11 @@ void ti8_run(bool p128, int64_t a8_0, int64_t sa_0, int64_t a8_1, int64_t sa_1, 
   a.N = N;
   a.SKG = skg;
   a.out_scale = out_scale;
+  if (skg > 1) {
+    const TI8Tail t = ti8_tail(K, N, r4_cus());
+    a.tail_f = t.f;
+    a.tail_s = t.s;
+  }
   hipStream_t st = (hipStream_t)stream;
   if (KB == 4) {
     if (p128) ti8_launch<4, kSBlk, kOutBf16, false>(a, N, skg, st);
@@ -628,7 +675,11 @@ void ti8_run(bool p128, int64_t a8_0, int64_t sa_0, int64_t a8_1, int64_t sa_1, 
     if (p128) ti8_launch<5, kSBlk, kOutBf16, false>(a, N, skg, st);
     else ti8_launch<5, kSCoarse, kOutBf16, false>(a, N, skg, st);
   }
-  if (skg > 1) r4d::launch_split_finish(a.ws, a.svh, a.c, M, N, skg, 1, out_scale, st);
+  if (a.tail_s > 1)
+    r4d::launch_split_finish(a.ws, a.svh + 128 * a.tail_f, (unsigned short*)a.c + 128 * a.tail_f, M, N - 128 * a.tail_f,
+                             a.tail_s, 1, out_scale, st, N);
+  else if (skg > 1)
+    r4d::launch_split_finish(a.ws, a.svh, a.c, M, N, skg, 1, out_scale, st);
   r4d::launch_ok(entry);
 }
 
@@ -746,6 +797,36 @@ void r4d_gemm_i8_dense_raw(int64_t a8, int64_t w8, int64_t c, int64_t ws, int64_
                            int SKG, int64_t stream) {
   dense_run(a8, 0, w8, 0, c, ws, tickets, M, K, N, SKG, 0, true, stream, "gemm_i8_dense_raw");
 }
+// This build's K split for the trellis int8 GEMM, fitted to a sweep of SKG 1..8 over the layer's shapes at TP 1 and 2 and
+// smaller ones: a 64-k step of one workgroup per CU takes 0.8 us (per-128: 1.1; the same picks), a split's finish and
+// partials 2 us and 0.045 us per workgroup-slice. Measured, SKG 1 / 2 / 4 (us): per-128 5120 x 16384 90.9 / 58.6 / 67.4,
+// 5120 x 8192 87.1 / 50.3 / 35.7; coarse 5120 x 17408 65.7 / 74.7 / 72.8, 5120 x 10240 64.3 / 40.6 / 47.3, 17408 x 5120
+// 194 / 103 / 59.8, 4096 x 2048 55.3 / 31.3 / 21.2 (SKG 8: 16.7). Above the CUs' number of groups SKG 2 names the tail split
+// (ti8_tail).
+int r4d_mi355x_trellis_i8_skg(int K, int N) {
+  const int G = N / 128, nkb = K / 128;
+  if (G <= 0 || nkb <= 0) return 1;
+  const int cus = r4_cus();
+  const TI8Tail t = ti8_tail(K, N, cus);
+  int best = 1;
+  double best_cost = 1e30;
+  for (int d = 1; d <= 8; d *= 2) {         // the split counts r4d_gemm_trellis_nt_i8_check allows (with skw 2)
+    if (nkb % (2 * d) && d > 1) continue;
+    const long long units = (long long)G * d;
+    const int steps = 2 * nkb / d;
+    double cost;
+    if (d > 1 && t.s > 1)
+      cost = 0.8 * ((double)(t.f / cus) * 2 * nkb + 2 * ((nkb + t.s - 1) / t.s)) + 2.0 + 0.045 * (G - t.f) * t.s;
+    else
+      cost = 0.8 * (double)((units + cus - 1) / cus) * steps + (d > 1 ? 2.0 + 0.045 * units : 0.0);
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = d;
+    }
+  }
+  return best;
+}
+
 // This build's K split for the dense int8 GEMM: the fewest slices (of at least 1024 k) that reach 128
 // workgroups -- the split that measured fastest at both config-4 shapes (1 at 5120 x 17408, 4 at 17408 x 5120).
 int r4d_mi355x_i8_skg(int K, int N) {

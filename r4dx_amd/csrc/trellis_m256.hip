@@ -431,8 +431,8 @@ __global__ __launch_bounds__(64 * kM2Waves, 1) void tq_m256_kernel(
 // 8.5 -> 7.3 us against a version that summed through LDS and stored two bytes per lane).
 constexpr int kFinRows = 16;   // rows of a workgroup
 __global__ __launch_bounds__(256) void tq_m256_finish(const float* __restrict__ ws, const float* __restrict__ svh,
-                                                      void* __restrict__ Cv, int M, int N, int SKG, int full,
-                                                      float out_scale) {
+                                                      void* __restrict__ Cv, int M, int N, int ldc, int SKG,
+                                                      int full, float out_scale) {
   const int lane = threadIdx.x & 63;
   const int r = blockIdx.y * kFinRows + (threadIdx.x >> 4), col = blockIdx.x * 128 + 8 * (lane & 15);
   const size_t sy = (size_t)M * N;
@@ -477,7 +477,7 @@ __global__ __launch_bounds__(256) void tq_m256_finish(const float* __restrict__ 
     }
   }
   if (!full) {
-    float* dst = (float*)Cv + (size_t)r * N + col;
+    float* dst = (float*)Cv + (size_t)r * ldc + col;
     *(r4f4_a4*)dst = (r4f4){v[0], v[1], v[2], v[3]};
     *(r4f4_a4*)(dst + 4) = (r4f4){v[4], v[5], v[6], v[7]};
     return;
@@ -486,7 +486,7 @@ __global__ __launch_bounds__(256) void tq_m256_finish(const float* __restrict__ 
   unsigned h[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) h[e] = r4_bf16_rn_sel((v[e] * sv[e]) * out_scale);
-  r4_store_u16<8>((unsigned short*)Cv + (size_t)r * N + col, h);
+  r4_store_u16<8>((unsigned short*)Cv + (size_t)r * ldc + col, h);
 }
 
 std::string m256_check(int M, int K, int N, int n_split, int KB, int SKG) {
@@ -589,8 +589,9 @@ void m256_run(int64_t a0, int64_t a1, int n_split, int64_t w, int64_t svh, int64
 }  // namespace
 
 void r4d::launch_split_finish(const float* ws, const float* svh, void* c, int M, int N, int SKG, int full,
-                              float out_scale, hipStream_t st) {
-  hipLaunchKernelGGL(tq_m256_finish, dim3(N / 128, M / kFinRows), dim3(256), 0, st, ws, svh, c, M, N, SKG, full, out_scale);
+                              float out_scale, hipStream_t st, int ldc) {
+  hipLaunchKernelGGL(tq_m256_finish, dim3(N / 128, M / kFinRows), dim3(256), 0, st, ws, svh, c, M, N, ldc ? ldc : N, SKG,
+                     full, out_scale);
 }
 
 // SK names the M <= 64 row this launch reproduces: 1 or 2 (0 means 1) is r4d_gemm_trellis_nt_m64's one-wave-per-pair

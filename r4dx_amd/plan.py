@@ -95,7 +95,7 @@ def plan_trellis_i8(N, K, kb, parts=1, part_n0=None, coarse=False):
     first = ""
     # the library's skg first, then smaller splits: (K / 128) must hold skw * skg, and a rank K such as 8704
     # (68 blocks = 4 * 17) takes skg 4 alone but no skw >= 2 beside it
-    skg = int(lib().r4d_mi355x_i8_skg(K, N))
+    skg = int(lib().r4d_mi355x_trellis_i8_skg(K, N))
     while skg >= 1:
         for skw in (2, 4, 8):
             msg = lib().r4d_gemm_trellis_nt_i8_check(PREFILL_M, K, N, n_split, kb, skw, skg)

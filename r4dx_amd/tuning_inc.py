@@ -74,7 +74,7 @@ def i8_row(N, K, KB, coarse):
 
 
 _HEAD = """// GENERATED by r4dx_amd/tuning_inc.py from libr4d_mi355x's planners (r4d_mi355x_trellis_gemv_skg,
-// r4d_mi355x_trellis_m256_skg, r4d_mi355x_i8_skg via r4dx_amd/plan.py); do not edit by hand.
+// r4d_mi355x_trellis_m256_skg, r4d_mi355x_trellis_i8_skg via r4dx_amd/plan.py); do not edit by hand.
 """
 
 
