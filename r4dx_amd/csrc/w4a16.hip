@@ -19,13 +19,13 @@
 // Dequant per dword (8 nibbles, nibble i at k = 16 s + 4 lh + {0, 8, 1, 9, 2, 10, 3, 11}[i]): masks
 // 0x000F000F and 0x00F000F0 of the dword and of the dword >> 8 pick the nibble pairs (0, 4), (1, 5),
 // (2, 6), (3, 7); one and-xor each gives the f16 bits of 1024 + q (the ^ 8 folded into the xor constant)
-// for a low nibble and of 1024 + 16 q for a high one; one packed f16 add of -(1024 + z), resp.
-// -(1024 + 16 z), gives q - z, resp. 16 (q - z), exactly. Pairs (0, 4), (2, 6) are k +0, +2, +1, +3
-// ("U", unscaled) and (1, 5), (3, 7) are k +8, +10, +9, +11 ("S", scaled by 16). A 64-k block is four
-// MFMAs of eight elements per lane: U of dwords (0, 1), U of (2, 3), S of (0, 1), S of (2, 3) -- each
-// inside one group of 32. The two chains are combined as (U + S / 16) * scale: the 1 / 16 undoes the
-// factor 16 exactly (a power of two). The A fragment of an MFMA is two runs of four k in that order,
-// staged in LDS with one row of zeros per (block, MFMA, k-half) for the lanes whose row is absent.
+// for a low nibble and of 1024 + 16 q for a high one; one packed f16 add of -(1024 + z), resp. one packed fma
+// by 1 / 16 and -(64 + z), gives q - z exactly. Pairs (0, 4), (2, 6) are k +0, +2, +1, +3 ("U") and (1, 5), (3, 7) are
+// k +8, +10, +9, +11 ("V"). A 64-k block is four MFMAs of eight elements per lane: U of dwords (0, 1), U of (2, 3), V of
+// (0, 1), V of (2, 3) -- each inside one group of 32; a group's MFMAs form one chain, whose sum takes the group's scale in
+// one fma per output. (With 16 (q - z) for the high nibbles a group had two chains and two fmas per output: above 8 rows
+// those 64 fmas per block at two row tiles weighed more than the MFMAs: 24 rows G = 32 216 -> 197 us, 64 rows 390 -> 366.) The A fragment of an MFMA is two runs of four k in
+// that order, staged in LDS with one row of zeros per (block, MFMA, k-half) for the lanes whose row is absent.
 //
 // Two MFMA forms. M <= 8: v_mfma_f32_16x16x32_f16 with rows (2 m + tile): lane (n, kq) holds the B data
 // of tile kq & 1, k-half kq >> 1, and A row rho is nonzero only where rho & 1 == kq & 1, so output row
@@ -52,32 +52,33 @@ constexpr int kWaves = 8;          // 8 waves = 256 output columns per workgroup
 // weight steps in flight per wave: 6 in the 16x16x32 form at G = 64 (measured faster there), else 4
 __host__ __device__ constexpr int w4_pf(int G, bool small) { return G == 64 && small ? 6 : 4; }
 constexpr int kNT = 2;             // cache policy of the weight loads: nontemporal (read once, streamed)
-constexpr int kLdsBudget = 40 * 1024;   // A chunk bytes per workgroup (four workgroups per CU)
+constexpr int kLdsBudget = 40 * 1024;   // A chunk bytes per workgroup (four workgroups per CU up to 8 rows)
 
-// 64-k blocks per A chunk for M rows (M + 1 staged): a multiple of pf, at most KB64 rounded up to one.
-__host__ __device__ inline int w4_chunk(int M, int KB64, int pf) {
-  int kc = kLdsBudget / (128 * (M + 1));
+// 64-k blocks per A chunk of `rows` staged rows (the last one zeros): a multiple of pf, at most KB64 rounded up to one.
+__host__ __device__ inline int w4_chunk(int rows, int KB64, int pf) {
+  int kc = kLdsBudget / (128 * rows);
   kc -= kc % pf;
   const int all = (KB64 + pf - 1) / pf * pf;
   return kc < all ? kc : all;
 }
 
-// B operand of MFMA c (0: U of dwords 0,1; 1: U of 2,3; 2: S of 0,1; 3: S of 2,3) from the dequantized
+// B operand of MFMA c (0: U of dwords 0,1; 1: U of 2,3; 2: V of 0,1; 3: V of 2,3) from the dequantized
 // halves: u[s] = (k +0,+2 ; +1,+3), v[s] = (k +8,+10 ; +9,+11).
 struct W4B {
   r4u2 u[4], v[4];
 };
-__device__ __forceinline__ void w4_dequant(const r4u4 w, const unsigned (&nz)[4], const unsigned (&nz16)[4], W4B& o) {
+__device__ __forceinline__ void w4_dequant(const r4u4 w, const unsigned (&nz)[4], const unsigned (&nzv)[4], W4B& o) {
+  const r4h2 inv16 = {(_Float16)0.0625f, (_Float16)0.0625f};
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
     const unsigned x = w[s], y = x >> 8;
     const unsigned p0 = (x & 0x000F000Fu) ^ 0x64086408u, p1 = (x & 0x00F000F0u) ^ 0x64806480u;
     const unsigned p2 = (y & 0x000F000Fu) ^ 0x64086408u, p3 = (y & 0x00F000F0u) ^ 0x64806480u;
-    const r4h2 z = __builtin_bit_cast(r4h2, nz[s]), z16 = __builtin_bit_cast(r4h2, nz16[s]);
+    const r4h2 z = __builtin_bit_cast(r4h2, nz[s]), zv = __builtin_bit_cast(r4h2, nzv[s]);
     o.u[s][0] = __builtin_bit_cast(unsigned, __builtin_bit_cast(r4h2, p0) + z);
     o.u[s][1] = __builtin_bit_cast(unsigned, __builtin_bit_cast(r4h2, p2) + z);
-    o.v[s][0] = __builtin_bit_cast(unsigned, __builtin_bit_cast(r4h2, p1) + z16);
-    o.v[s][1] = __builtin_bit_cast(unsigned, __builtin_bit_cast(r4h2, p3) + z16);
+    o.v[s][0] = __builtin_bit_cast(unsigned, __builtin_elementwise_fma(__builtin_bit_cast(r4h2, p1), inv16, zv));
+    o.v[s][1] = __builtin_bit_cast(unsigned, __builtin_elementwise_fma(__builtin_bit_cast(r4h2, p3), inv16, zv));
   }
 }
 __device__ __forceinline__ r4h8 w4_bop(const W4B& b, int c) {
@@ -88,13 +89,10 @@ __device__ __forceinline__ r4h8 w4_bop(const W4B& b, int c) {
 // k offset (in the 64-k block, before 4 lh) of the first run of MFMA c's A fragment; the second run is +16
 __host__ __device__ constexpr int w4_run_k(int c) { return c == 0 ? 0 : c == 1 ? 32 : c == 2 ? 8 : 40; }
 
-// (f16 -(1024 + z), f16 -(1024 + 16 z)) pairs of one Wsz word: -(1024 + 16 z) = 16 (-(1024 + z)) + 15360,
-// exact in f16 (integers below 2048)
-__device__ __forceinline__ void w4_zeros(unsigned szw, unsigned& nz, unsigned& nz16) {
+// (f16 -(1024 + z), f16 -(64 + z)) pairs of one Wsz word: -(64 + z) = -(1024 + z) + 960, exact in f16 (integers below 2048)
+__device__ __forceinline__ void w4_zeros(unsigned szw, unsigned& nz, unsigned& nzv) {
   nz = __builtin_amdgcn_perm(szw, szw, 0x03020302u);
-  nz16 = __builtin_bit_cast(unsigned, __builtin_elementwise_fma(__builtin_bit_cast(r4h2, nz),
-                                                                (r4h2){(_Float16)16.0f, (_Float16)16.0f},
-                                                                (r4h2){(_Float16)15360.0f, (_Float16)15360.0f}));
+  nzv = __builtin_bit_cast(unsigned, __builtin_bit_cast(r4h2, nz) + (r4h2){(_Float16)960.0f, (_Float16)960.0f});
 }
 
 // ---- argmax ------------------------------------------------------------------------------------------
@@ -248,21 +246,27 @@ __device__ __forceinline__ void w4_store_argmax(const Acc (&acc)[SMALL ? 1 : MT]
   }
 }
 
-// SMALL: the 16x16x32 form (M <= 8). MT: row tiles of 32 in the 32x32x16 form.
+// MR: the form's rows, the next of {1, 2, 4, 8, 32, 64} from M on. SMALL (MR <= 8): the 16x16x32 form, whose MR + 1 staged rows
+// have a constant stride, so fragment addresses are one register plus immediates and the staging divides nothing (with M +
+// 1 rows, G = 32, 1 / 4 / 8 rows: 144 / 161 / 156 -> 135 / 148 / 151 us at 5120 x 248320 with argmax; at G = 64 up to 2 %).
+// Above that MT row tiles of 32 in the 32x32x16 form with M + 1 staged rows (padded rows shorten the chunks: 2 to 5 % slower).
 // AM (with OUTF): the fused per-row argmax of the logits (AmFused).
-template <int G, bool SMALL, int MT, bool OUTF, bool AM>
-__global__ __launch_bounds__(64 * kWaves) void w4_kernel(const unsigned short* __restrict__ A,
+template <int G, int MR, bool OUTF, bool AM>
+__global__ __launch_bounds__(64 * kWaves, MR <= 8 ? (G == 32 ? 8 : 6) : 1) void w4_kernel(
+                                                          const unsigned short* __restrict__ A,
                                                           const unsigned* __restrict__ Wq,
                                                           const unsigned* __restrict__ Wsz,
                                                           void* __restrict__ Cv, int M, int K, int N, AmFused af) {
   static_assert(!AM || OUTF, "the fused argmax reads fp32 logits");
+  constexpr bool SMALL = MR <= 8;
+  constexpr int MT = MR <= 32 ? 1 : 2;
   extern __shared__ r4u4 alds[];   // chunk fragments [kb][c][lh][M] of 8 halves, then a zero block
   const int lane = threadIdx.x & 63;
   const int KB64 = K >> 6, groups = K / G;
   const int tiles = N >> 4;
   constexpr int kPF = w4_pf(G, SMALL);
-  const int KC = w4_chunk(M, KB64, kPF);
-  const int M1 = M + 1;                        // staged rows: row M is zero
+  const int M1 = SMALL ? MR + 1 : M + 1;       // staged rows: the last one is zero
+  const int KC = w4_chunk(M1, KB64, kPF);
   int t0 = (blockIdx.x * kWaves + (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * 2;
   const bool live = t0 < tiles;
   if (!live) t0 = tiles - 1;                   // a spare wave streams the last tile and stores nothing
@@ -292,31 +296,45 @@ __global__ __launch_bounds__(64 * kWaves) void w4_kernel(const unsigned short* _
     } else {
       m = i * 32 + (lane & 31); h = lh; ok = m < M;
     }
-    a_lane[i] = (unsigned)((h * M1 + (ok ? m : M)) * 16);
+    a_lane[i] = (unsigned)((h * M1 + (ok ? m : M1 - 1)) * 16);
   }
-  const unsigned kb_stride = 8u * (unsigned)M1 * 16u;   // bytes per 64-k block in the chunk
+  const unsigned kbStride = 8u * (unsigned)M1 * 16u;   // bytes per 64-k block in the chunk
   auto afrag = [&](int i, int kbl, int c) -> r4h8 {
-    const unsigned off = (unsigned)kbl * kb_stride + (unsigned)c * 2u * M1 * 16u + a_lane[i];
-    return __builtin_bit_cast(r4h8, *(const r4u4*)((const char*)alds + off));
+    return __builtin_bit_cast(r4h8, *(const r4u4*)((const char*)alds + (a_lane[i] + (unsigned)kbl * kbStride) +
+                                                   (unsigned)c * 2u * (unsigned)M1 * 16u));
   };
   // stage 64-k blocks [kb0, kb0 + KC) of A: fragment ((kbl * 4 + c) * 2 + h) * M1 + m holds
-  // A[m][64 kb + run_k(c) + 4 h + {0, 2, 1, 3, 16, 18, 17, 19}] (row M: zeros)
+  // A[m][64 kb + run_k(c) + 4 h + {0, 2, 1, 3, 16, 18, 17, 19}]
+  auto frag_of = [&](const unsigned short* src) {
+    const r4u2 lo = *(const r4u2_a2*)src, hi = *(const r4u2_a2*)(src + 16);
+    return (r4u4){__builtin_amdgcn_perm(lo[1], lo[0], 0x05040100u), __builtin_amdgcn_perm(lo[1], lo[0], 0x07060302u),
+                  __builtin_amdgcn_perm(hi[1], hi[0], 0x05040100u), __builtin_amdgcn_perm(hi[1], hi[0], 0x07060302u)};
+  };
   auto stage = [&](int kb0) {
-    const int n = min(KC, KB64 - kb0) * 8 * M1;
-    for (int i = threadIdx.x; i < n; i += 64 * kWaves) {
-      const int m = i % M1, rest = i / M1, h = rest & 1, c = (rest >> 1) & 3, kbl = rest >> 3;
-      r4u4 v = {0u, 0u, 0u, 0u};
-      if (m < M) {
-        const unsigned short* src = A + (size_t)m * K + 64 * (kb0 + kbl) + w4_run_k(c) + 4 * h;
-        const r4u2 lo = *(const r4u2*)src, hi = *(const r4u2*)(src + 16);
-        v[0] = __builtin_amdgcn_perm(lo[1], lo[0], 0x05040100u);
-        v[1] = __builtin_amdgcn_perm(lo[1], lo[0], 0x07060302u);
-        v[2] = __builtin_amdgcn_perm(hi[1], hi[0], 0x05040100u);
-        v[3] = __builtin_amdgcn_perm(hi[1], hi[0], 0x07060302u);
+    const int nb = min(KC, KB64 - kb0);
+    if constexpr (SMALL) {
+      // thread t takes row t mod MR, (c, h) = the next three bits and every kS-th block; rows past M are neither staged nor
+      // read, the zero row is written once (below)
+      constexpr int kS = 64 * kWaves / (8 * MR);
+      int t = threadIdx.x;
+      asm volatile("" : "+v"(t));                // the thread's addresses are formed here, not kept through the k loop
+      const int sm = t % MR, sch = (t / MR) & 7;
+      const unsigned short* const sa = A + (size_t)min(sm, M - 1) * K + w4_run_k(sch >> 1) + 4 * (sch & 1);
+      r4u4* const sd = alds + sch * M1 + sm;
+      if (sm < M) {
+#pragma unroll 2
+        for (int kbl = t / (8 * MR); kbl < nb; kbl += kS) sd[kbl * 8 * M1] = frag_of(sa + 64 * (kb0 + kbl));
       }
-      alds[i] = v;
+    } else {
+      for (int i = threadIdx.x; i < nb * 8 * M1; i += 64 * kWaves) {
+        const int m = i % M1, rest = i / M1, h = rest & 1, c = (rest >> 1) & 3, kbl = rest >> 3;
+        alds[i] = m < M ? frag_of(A + (size_t)m * K + 64 * (kb0 + kbl) + w4_run_k(c) + 4 * h) : (r4u4){0u, 0u, 0u, 0u};
+      }
     }
   };
+  if constexpr (SMALL) {
+    for (int i = threadIdx.x; i < KC * 8; i += 64 * kWaves) alds[i * M1 + MR] = (r4u4){0u, 0u, 0u, 0u};
+  }
 
   using Acc = typename std::conditional<SMALL, r4f4, r4f16>::type;
   Acc acc[NA];
@@ -339,14 +357,14 @@ __global__ __launch_bounds__(64 * kWaves) void w4_kernel(const unsigned short* _
     s.w = __builtin_bit_cast(r4u4, __builtin_amdgcn_raw_buffer_load_b128(wr, wlane + (unsigned)kc * 512u, 0, kNT));
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
-      const unsigned go = (unsigned)(NG * kc + g) * 64u;
+      const int go = (NG * kc + g) * 64;
       if constexpr (COOP) {
-        if (g == 0) s.sz[0] = __builtin_amdgcn_raw_buffer_load_b32(sr, coop_base + (unsigned)(NG * kc) * 64u, 0, kNT);
+        if (g == 0) s.sz[0] = __builtin_amdgcn_raw_buffer_load_b32(sr, coop_base, go, kNT);
       } else if constexpr (SMALL) {
-        s.sz[2 * g] = __builtin_amdgcn_raw_buffer_load_b32(sr, st0 + go, 0, kNT);
-        s.sz[2 * g + 1] = __builtin_amdgcn_raw_buffer_load_b32(sr, st1 + go, 0, kNT);
+        s.sz[2 * g] = __builtin_amdgcn_raw_buffer_load_b32(sr, st0, go, kNT);
+        s.sz[2 * g + 1] = __builtin_amdgcn_raw_buffer_load_b32(sr, st1, go, kNT);
       } else {
-        s.sz[g] = __builtin_amdgcn_raw_buffer_load_b32(sr, sown + go, 0, kNT);
+        s.sz[g] = __builtin_amdgcn_raw_buffer_load_b32(sr, sown + (unsigned)go, 0, kNT);
       }
     }
   };
@@ -366,48 +384,45 @@ __global__ __launch_bounds__(64 * kWaves) void w4_kernel(const unsigned short* _
       __device__ unsigned operator[](int i) const { return p[i]; }
     };
     const struct { SzView sz; } s{SzView{COOP ? szl : s0.sz}};
-    unsigned nz[4], nz16[4];
+    unsigned nz[4], nzv[4];
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
       const unsigned own = SMALL ? (own1 ? s.sz[2 * g + 1] : s.sz[2 * g]) : s.sz[g];
       unsigned a, b;
       w4_zeros(own, a, b);
 #pragma unroll
-      for (int q = 0; q < 4 / NG; ++q) { nz[g * (4 / NG) + q] = a; nz16[g * (4 / NG) + q] = b; }
+      for (int q = 0; q < 4 / NG; ++q) { nz[g * (4 / NG) + q] = a; nzv[g * (4 / NG) + q] = b; }
     }
     W4B bq;
-    w4_dequant(s0.w, nz, nz16, bq);
+    w4_dequant(s0.w, nz, nzv, bq);
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
-      // group g: G = 64 -> U chain (c 0, 1), S chain (c 2, 3); G = 32 -> g 0: c 0 / 2, g 1: c 1 / 3
+      // group g's chain: G = 64 -> c 0, 2, 1, 3; G = 32 -> c g, 2 + g. At 8 rows and fewer, where the wave has no other MFMAs
+      // to fill in, G = 64 runs as two chains added: one of four dependent MFMAs was 1.5 % slower.
+      constexpr int kCh = G == 64 && SMALL ? 2 : 1;
 #pragma unroll
       for (int i = 0; i < NA; ++i) {
-        Acc tu, ts;
+        Acc t[kCh];
+#pragma unroll
+        for (int u = 0; u < 4 / NG; ++u) {
+          const int c = G == 64 ? (u & 1) * 2 + (u >> 1) : g + 2 * u, ch = u & (kCh - 1);
+          const Acc t0 = u < kCh ? Acc{} : t[ch];
+          if constexpr (SMALL) t[ch] = __builtin_amdgcn_mfma_f32_16x16x32_f16(afrag(i, kbl, c), w4_bop(bq, c), t0, 0, 0, 0);
+          else t[ch] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afrag(i, kbl, c), w4_bop(bq, c), t0, 0, 0, 0);
+        }
         if constexpr (SMALL) {
-          tu = __builtin_amdgcn_mfma_f32_16x16x32_f16(afrag(i, kbl, G == 64 ? 0 : g), w4_bop(bq, G == 64 ? 0 : g), Acc{}, 0, 0, 0);
-          ts = __builtin_amdgcn_mfma_f32_16x16x32_f16(afrag(i, kbl, G == 64 ? 2 : 2 + g), w4_bop(bq, G == 64 ? 2 : 2 + g), Acc{}, 0, 0, 0);
-          if constexpr (G == 64) {
-            tu = __builtin_amdgcn_mfma_f32_16x16x32_f16(afrag(i, kbl, 1), w4_bop(bq, 1), tu, 0, 0, 0);
-            ts = __builtin_amdgcn_mfma_f32_16x16x32_f16(afrag(i, kbl, 3), w4_bop(bq, 3), ts, 0, 0, 0);
-          }
           // output rows 4 (lane >> 4) + e = 2 m + t: tile t = e & 1 (rows m >= M have zero A and stay 0)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const float sc = r4_f16_to_f32((unsigned short)(s.sz[2 * g + (e & 1)] & 0xFFFFu));
-            acc[i][e] = __builtin_fmaf(__builtin_fmaf(ts[e], 0.0625f, tu[e]), sc, acc[i][e]);
+            acc[i][e] = __builtin_fmaf(kCh == 2 ? t[0][e] + t[kCh - 1][e] : t[0][e], sc, acc[i][e]);
           }
         } else {
-          tu = __builtin_amdgcn_mfma_f32_32x32x16_f16(afrag(i, kbl, G == 64 ? 0 : g), w4_bop(bq, G == 64 ? 0 : g), Acc{}, 0, 0, 0);
-          ts = __builtin_amdgcn_mfma_f32_32x32x16_f16(afrag(i, kbl, G == 64 ? 2 : 2 + g), w4_bop(bq, G == 64 ? 2 : 2 + g), Acc{}, 0, 0, 0);
-          if constexpr (G == 64) {
-            tu = __builtin_amdgcn_mfma_f32_32x32x16_f16(afrag(i, kbl, 1), w4_bop(bq, 1), tu, 0, 0, 0);
-            ts = __builtin_amdgcn_mfma_f32_32x32x16_f16(afrag(i, kbl, 3), w4_bop(bq, 3), ts, 0, 0, 0);
-          }
           const float sc = r4_f16_to_f32((unsigned short)(s.sz[g] & 0xFFFFu));
           // only the rows this launch has: row = (e / 4) * 8 + lh * 4 + e % 4
 #pragma unroll
           for (int e = 0; e < 16; ++e)
-            if (i * 32 + (e >> 2) * 8 < M) acc[i][e] = __builtin_fmaf(__builtin_fmaf(ts[e], 0.0625f, tu[e]), sc, acc[i][e]);
+            if (i * 32 + (e >> 2) * 8 < M) acc[i][e] = __builtin_fmaf(t[0][e], sc, acc[i][e]);
         }
       }
     }
@@ -495,14 +510,20 @@ void w4_launch(int64_t a, int64_t wq, int64_t wsz, int64_t c, int M, int K, int 
   const int tiles = N / 16;
   const int waves = (tiles + 1) / 2;
   dim3 grid((waves + kWaves - 1) / kWaves), block(64 * kWaves);
-  size_t smem = (size_t)w4_chunk(M, K / 64, w4_pf(G, M <= 8)) * 8 * (M + 1) * 16;
-  if (AM && smem < w4_am_lds(M <= 8)) smem = w4_am_lds(M <= 8);
-  auto Ap = (const unsigned short*)a;
-  auto Wp = (const unsigned*)wq;
-  auto Sp = (const unsigned*)wsz;
-  if (M <= 8) hipLaunchKernelGGL((w4_kernel<G, true, 1, OUTF, AM>), grid, block, smem, st, Ap, Wp, Sp, (void*)c, M, K, N, af);
-  else if (M <= 32) hipLaunchKernelGGL((w4_kernel<G, false, 1, OUTF, AM>), grid, block, smem, st, Ap, Wp, Sp, (void*)c, M, K, N, af);
-  else hipLaunchKernelGGL((w4_kernel<G, false, 2, OUTF, AM>), grid, block, smem, st, Ap, Wp, Sp, (void*)c, M, K, N, af);
+  auto go = [&](auto mr) {
+    constexpr int MR = decltype(mr)::value;
+    const int rows = MR <= 8 ? MR + 1 : M + 1;
+    size_t smem = (size_t)w4_chunk(rows, K / 64, w4_pf(G, MR <= 8)) * 8 * rows * 16;
+    if (AM && smem < w4_am_lds(MR <= 8)) smem = w4_am_lds(MR <= 8);
+    hipLaunchKernelGGL((w4_kernel<G, MR, OUTF, AM>), grid, block, smem, st, (const unsigned short*)a, (const unsigned*)wq,
+                       (const unsigned*)wsz, (void*)c, M, K, N, af);
+  };
+  if (M <= 1) go(std::integral_constant<int, 1>());
+  else if (M <= 2) go(std::integral_constant<int, 2>());
+  else if (M <= 4) go(std::integral_constant<int, 4>());
+  else if (M <= 8) go(std::integral_constant<int, 8>());
+  else if (M <= 32) go(std::integral_constant<int, 32>());
+  else go(std::integral_constant<int, 64>());
 }
 
 void w4_run(int group, int64_t a, int64_t wq, int64_t wsz, int64_t c, int M, int K, int N, bool outf,
