@@ -13,9 +13,17 @@ def _p(t):
     return 0 if t is None else t.data_ptr()
 
 
+# The current stream's handle without a torch.cuda.Stream object around it: a launch of a few microseconds paid 2.8 us for
+# the object and 0.2 us for the handle. (Where torch has no such entry, the object.)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(stream=None):
-    s = torch.cuda.current_stream() if stream is None else stream
-    return s.cuda_stream
+    if stream is not None:
+        return stream.cuda_stream
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 class TicketBuffer:
