@@ -116,7 +116,7 @@ struct TqOut {
 // the ticket flag.
 constexpr size_t tq_end_lds_flag(int MT, int NPW, int SK, int M) {
   const size_t parts = (size_t)(SK - 1) * NPW * 8 * MT * 64 * 4;
-  const size_t sums = MT > 1 || NPW == 4 ? (size_t)M * NPW * 32 * 4 : 0;
+  const size_t sums = MT > 1 || NPW >= 2 ? (size_t)M * NPW * 32 * 4 : 0;
   return parts > sums ? parts : sums;
 }
 constexpr size_t tq_end_lds(int MT, int NPW, int SK, int M) { return tq_end_lds_flag(MT, NPW, SK, M) + 16; }
@@ -132,7 +132,8 @@ constexpr size_t tq_end_lds(int MT, int NPW, int SK, int M) { return tq_end_lds_
 //     every slice of a batch of 8 requested before any is added.
 // Each 32-lane half of a wave then owns one row's 128 sums, 4 adjacent columns per lane, from the slice sum to the
 // store (r4_fwht128_rows): no LDS copy of the slice sums, no stage through the LDS crossbar and one 8-byte store per lane.
-template <int MT, int NPW, int SK>
+// STAGE: also one row tile above 8 rows goes through LDS.
+template <int MT, int NPW, int SK, bool STAGE = false>
 __device__ __forceinline__ void tq_finish(const r4f4 (&acc)[MT][2], unsigned char* lds, const TqOut& o, int group, int pair,
                                           int ks, int ky) {
   constexpr int NT = 64 * NPW * SK;
@@ -160,11 +161,12 @@ __device__ __forceinline__ void tq_finish(const r4f4 (&acc)[MT][2], unsigned cha
     return;
   }
   const bool in_block = NPW == 4 && SK == 1 && SKG == 1;   // the workgroup holds its whole group
-  constexpr bool kStaged = MT > 1;              // the partials pass through LDS and leave as whole 16-byte row pieces
+  // the partials pass through LDS and leave as whole 16-byte row pieces (up to 8 rows their few 4-byte stores are as fast)
+  const bool staged = MT > 1 || (STAGE && M > 8);
   constexpr int kCols = 32 * NPW;               // the workgroup's columns
   const unsigned sy4 = (unsigned)M * (unsigned)N * 4u;
   const r4_rsrc wsr = r4_make_rsrc(o.ws, (unsigned)SKG * sy4);
-  if (in_block || kStaged) {
+  if (in_block || staged) {
     if constexpr (SK > 1) __syncthreads();      // the part accumulators have been read
     const int lcol0 = gcol0 & (kCols - 1);
     if (ks == 0) {
@@ -182,7 +184,7 @@ __device__ __forceinline__ void tq_finish(const r4f4 (&acc)[MT][2], unsigned cha
     __syncthreads();
   }
   if (!in_block) {
-    if constexpr (kStaged) {
+    if (staged) {
       const unsigned base = (unsigned)ky * sy4 + (unsigned)(n0 + (kCols == 128 ? 0 : (pair * 32) & (128 - kCols))) * 4u;
       for (int it = (int)threadIdx.x; it < M * (kCols / 4); it += NT) {
         const int r = it / (kCols / 4), cq = it & (kCols / 4 - 1);

@@ -20,17 +20,7 @@
 
 namespace {
 
-// A row's two fragments (h = 0, 1) of one k-tile from the row buffer at byte offset off:
-// k 16kt + {0..3, 8..11} and {4..7, 12..15}.
-__device__ __forceinline__ void load_a(r4h8 (&af)[2], r4_rsrc r, unsigned off) {
-  const r4u4 lo = __builtin_bit_cast(r4u4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-  const r4u4 hi = __builtin_bit_cast(r4u4, __builtin_amdgcn_raw_buffer_load_b128(r, off + 16, 0, 0));
-  const r4u4 f0 = {lo[0], lo[1], hi[0], hi[1]}, f1 = {lo[2], lo[3], hi[2], hi[3]};
-  af[0] = __builtin_bit_cast(r4h8, f0);
-  af[1] = __builtin_bit_cast(r4h8, f1);
-}
-
-// Same, for the plain pointer form (the reconstruct kernel).
+// A lane's words through a plain pointer (the reconstruct kernel).
 template <int KB>
 __device__ __forceinline__ void load_words_ptr(Words<KB>& s, const unsigned* __restrict__ blk, int t, int c) {
   const unsigned* tile = blk + t * 8 * KB;
@@ -49,9 +39,9 @@ __device__ __forceinline__ void load_words_ptr(Words<KB>& s, const unsigned* __r
 // XF > 0: A0 is the raw input x [M][K] (XF 1: f16, 2: bf16) and the workgroup stages its own slice of the
 // transformed A = f16(FWHT128(fp32(x) * suh) * xscale) (suh of the group's column part) straight into LDS --
 // the arithmetic of r4dx_trellis_input_*, so A is bit-identical to the unfused path's.
-// The decode forms (one row tile, A in LDS) ask for 6 waves per SIMD: their register need lies just above that budget.
-template <int KB, int MT, int NPW, int SK, bool ALDS, int XF, bool WQ = false>
-__global__ __launch_bounds__(64 * NPW * SK, MT == 1 && ALDS && SK == 4 && XF == 0 && !WQ ? 6 : 1) void tq_gemv_kernel(
+// The decode forms (one row tile) ask for 6 waves per SIMD: their register need lies just above that budget.
+template <int KB, int MT, int NPW, int SK, int XF, bool WQ = false>
+__global__ __launch_bounds__(64 * NPW * SK, MT == 1 && SK == 4 && !WQ ? 6 : 1) void tq_gemv_kernel(
     const R4AParts ap,
     const unsigned* __restrict__ W, const float* __restrict__ svh, void* __restrict__ Cv,
     float* __restrict__ ws, unsigned* __restrict__ tickets, int M, int K, int N, int SKG, int full,
@@ -88,7 +78,7 @@ __global__ __launch_bounds__(64 * NPW * SK, MT == 1 && ALDS && SK == 4 && XF == 
   const int ktl_pad = SK * nsw * 4;            // k-tiles the LDS copy of A covers (zero past ktw)
   const unsigned mmag = r4_div_magic((unsigned)M);
 
-  // LDS: the A slice (ALDS) + its zero block while the k loop runs; after it (every wave past the barrier that ends
+  // LDS: the A slice + its zero block while the k loop runs; after it (every wave past the barrier that ends
   // the loop), the same bytes hold the unit's end (tq_end_lds). The launch asks for the larger of the two.
   r4u4* alds = lds_raw;
   float* part_acc = (float*)lds_raw;
@@ -98,35 +88,23 @@ __global__ __launch_bounds__(64 * NPW * SK, MT == 1 && ALDS && SK == 4 && XF == 
   const LaneWords<KB> lw(q, t, c);
   constexpr unsigned kStepBytes = 4 * BLK * 4;
   // A: LDS byte address of this lane's fragment pair at step 0 and its per-step stride (rows >= M
-  // read the zero block with stride 0); or, from global memory, a buffer over A with the row offset.
+  // read the zero block with stride 0)
   unsigned a_off[MT], a_stride[MT];
   const r4_rsrc ar = r4_make_rsrc(A, (unsigned)((size_t)M * K * 2));
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     const int r = i * 16 + mrow;
-    if constexpr (ALDS) {
-      a_off[i] = r < M ? (unsigned)(((st_beg * 4 + q) * M + r) * 32) : (unsigned)(ktl_pad * M * 32);
-      a_stride[i] = r < M ? (unsigned)(4 * M * 32) : 0u;
-    } else {
-      a_off[i] = r < M ? (unsigned)((size_t)r * K * 2 + (size_t)(kt0 + st_beg * 4 + q) * 32) : 0x80000000u;
-      a_stride[i] = 4 * 32;
-    }
+    a_off[i] = r < M ? (unsigned)(((st_beg * 4 + q) * M + r) * 32) : (unsigned)(ktl_pad * M * 32);
+    a_stride[i] = r < M ? (unsigned)(4 * M * 32) : 0u;
   }
 
   struct St {
     Words<KB> w;
-    r4h8 a[ALDS ? 1 : MT][2];
   };
   // Step s of this wave (clamped to its last step, so a prefetch past the end re-reads a cached
   // line instead of another wave's weights).
   auto load = [&](St& s, int sidx) {
-    const int sc = min(sidx, nst - 1);
-    load_words<KB, XF == 0>(s.w, wr, lw, (unsigned)(st_beg + sc) * kStepBytes);
-    if constexpr (!ALDS) {
-      const bool ok = (st_beg + sc) * 4 + q < ktw;
-#pragma unroll
-      for (int i = 0; i < MT; ++i) load_a(s.a[i], ar, ok ? a_off[i] + (unsigned)sc * a_stride[i] : 0x80000000u);
-    }
+    load_words<KB, XF == 0>(s.w, wr, lw, (unsigned)(st_beg + min(sidx, nst - 1)) * kStepBytes);
   };
   r4f4 acc[MT][2];
 #pragma unroll
@@ -135,14 +113,9 @@ __global__ __launch_bounds__(64 * NPW * SK, MT == 1 && ALDS && SK == 4 && XF == 
     r4h8 af[MT][2];
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
-      if constexpr (ALDS) {
-        const r4u4* p = (const r4u4*)((const char*)alds + a_off[i] + (unsigned)sidx * a_stride[i]);
-        af[i][0] = __builtin_bit_cast(r4h8, p[0]);
-        af[i][1] = __builtin_bit_cast(r4h8, p[1]);
-      } else {
-        af[i][0] = s.a[i][0];
-        af[i][1] = s.a[i][1];
-      }
+      const r4u4* p = (const r4u4*)((const char*)alds + a_off[i] + (unsigned)sidx * a_stride[i]);
+      af[i][0] = __builtin_bit_cast(r4h8, p[0]);
+      af[i][1] = __builtin_bit_cast(r4h8, p[1]);
     }
     unsigned d[2][2][4];
     if constexpr (XF == 0) {
@@ -217,8 +190,8 @@ __global__ __launch_bounds__(64 * NPW * SK, MT == 1 && ALDS && SK == 4 && XF == 
 #pragma unroll
     for (int i = 0; i < PF; ++i) load(ring[i], i);
   };
-  if constexpr (!(ALDS && XF == 0)) load_ring();
-  if constexpr (ALDS && XF > 0) {
+  if constexpr (XF > 0) load_ring();
+  if constexpr (XF > 0) {
     // A = f16(FWHT128(fp32(x) * suh) * xscale) (r4_fwht128_wave_pairs: the same fp32 operations per element
     // as r4dx_trellis_input_*), each lane's two adjacent k written as one dword to its fragment slot --
     // element k16 of k-tile ktl sits at half (k16 >> 3) + 2 ((k16 >> 2) & 1) of the 32-byte (ktl, row)
@@ -251,7 +224,7 @@ __global__ __launch_bounds__(64 * NPW * SK, MT == 1 && ALDS && SK == 4 && XF == 
     }
     if (threadIdx.x < 8) ah[(size_t)ktl_pad * M * 8 + threadIdx.x] = 0u;
     __syncthreads();
-  } else if constexpr (ALDS) {
+  } else {
     // chunk (ktl, row, j): k 16 (kt0 + ktl) + 8j .. + 8 of A[row] -> halves of fragments h = 0, 1;
     // k-tiles past the slice are zero, and so is the 32-byte block after the copy (rows >= M read it).
     // kStageU chunks per thread per pass, all loads issued before any is written: one memory round trip
@@ -325,7 +298,7 @@ __global__ __launch_bounds__(64 * NPW * SK, MT == 1 && ALDS && SK == 4 && XF == 
   }
 
   // The A slice is dead once every wave has left the loop: the combine, the sums and the reduce runs reuse its bytes.
-  if constexpr (ALDS) __syncthreads();
+  __syncthreads();
   tq_combine<MT, NPW, SK>(acc, part_acc, pl, ks, lane);
 
   if (probe) {
@@ -334,7 +307,7 @@ __global__ __launch_bounds__(64 * NPW * SK, MT == 1 && ALDS && SK == 4 && XF == 
   }
 
   const TqOut out{svh, Cv, ws, tickets, M, N, SKG, full, out_scale};
-  tq_finish<MT, NPW, SK>(acc, (unsigned char*)lds_raw, out, group, pair, ks, ky);
+  tq_finish<MT, NPW, SK, NPW == 2 && XF == 0>(acc, (unsigned char*)lds_raw, out, group, pair, ks, ky);
 }
 
 // One wave per (tile pair, 4-k-tile step): every lane decodes its 32 weights with the GEMM's own
@@ -413,9 +386,9 @@ __global__ __launch_bounds__(256) void tq_wscale_kernel(const unsigned* __restri
 
 // Dynamic LDS of one launch.
 size_t gemv_ktl_pad(int SK, int ktw) { return (size_t)SK * ((((ktw + 3) >> 2) + SK - 1) / SK) * 4; }
-// The A slice (ALDS) and, after the k loop, in the same bytes: the unit's end.
-size_t gemv_lds(int MT, int NPW, int SK, bool alds, int ktw, int M) {
-  const size_t a = alds ? gemv_ktl_pad(SK, ktw) * M * 32 + 32 : 0;
+// The A slice and, after the k loop, in the same bytes: the unit's end.
+size_t gemv_lds(int MT, int NPW, int SK, int ktw, int M) {
+  const size_t a = gemv_ktl_pad(SK, ktw) * M * 32 + 32;
   const size_t tail = tq_end_lds(MT, NPW, SK, M);
   return a > tail ? a : tail;
 }
@@ -439,23 +412,21 @@ GemvForm gemv_form(int M, int N, int SKG, bool have_ws, bool sk1, bool xf = fals
   else { f.NPW = M == 1 && !(xf && N >= 8192) ? 1 : 2; f.SK = 4; }
   return f;
 }
-// The LDS bytes of a launch of that form (alds: A staged in LDS, forced by the fused transform).
-size_t gemv_form_lds(int M, int K, int N, int SKG, bool have_ws, bool sk1, bool xf) {
-  const GemvForm f = gemv_form(M, N, SKG, have_ws, sk1, xf);
-  const int ktw = K / 16 / SKG;
-  const bool alds = xf || gemv_ktl_pad(f.SK, ktw) * M * 32 <= kAldsMax;
-  return gemv_lds(f.MT, f.NPW, f.SK, alds, ktw, M);
+// The LDS bytes of a fused-transform launch.
+size_t gemv_xf_lds(int M, int K, int N, int SKG, bool have_ws) {
+  const GemvForm f = gemv_form(M, N, SKG, have_ws, false, true);
+  return gemv_lds(f.MT, f.NPW, f.SK, K / 16 / SKG, M);
 }
 
-template <int KB, int MT, int NPW, int SK, bool ALDS, int XF, bool WQ = false>
+template <int KB, int MT, int NPW, int SK, int XF, bool WQ = false>
 void launch_gemv(const r4d_gemv_args& a) {
   dim3 grid(a.N / 32 / NPW, a.SKG), block(64 * NPW * SK);
   const int ktw = a.K / 16 / a.SKG;
-  const size_t smem = gemv_lds(MT, NPW, SK, ALDS, ktw, a.M);
+  const size_t smem = gemv_lds(MT, NPW, SK, ktw, a.M);
   if (smem > 160 * 1024) r4d::fail("gemm_trellis_nt_m64", "LDS request above 160 KiB");
   static std::atomic<unsigned long long> lds_set{0};
   if (smem > 64 * 1024)
-    r4d::allow_lds((const void*)tq_gemv_kernel<KB, MT, NPW, SK, ALDS, XF, WQ>, lds_set, "gemm_trellis_nt_m64");
+    r4d::allow_lds((const void*)tq_gemv_kernel<KB, MT, NPW, SK, XF, WQ>, lds_set, "gemm_trellis_nt_m64");
   const R4AParts ap = r4_parts((const void*)a.a0, (const void*)a.a1, a.n_split, (const void*)a.a2, a.n_end1,
                                (const void*)a.a3, a.n_end2);
   R4SParts sp;
@@ -463,7 +434,7 @@ void launch_gemv(const r4d_gemv_args& a) {
   sp.s[1] = (const float*)(a.suh1 ? a.suh1 : a.suh0);
   sp.s[2] = a.suh2 ? (const float*)a.suh2 : sp.s[1];
   sp.s[3] = a.suh3 ? (const float*)a.suh3 : sp.s[2];
-  hipLaunchKernelGGL((tq_gemv_kernel<KB, MT, NPW, SK, ALDS, XF, WQ>), grid, block, smem, (hipStream_t)a.stream, ap,
+  hipLaunchKernelGGL((tq_gemv_kernel<KB, MT, NPW, SK, XF, WQ>), grid, block, smem, (hipStream_t)a.stream, ap,
                      (const unsigned*)a.w, (const float*)a.svh, (void*)a.c, (float*)a.ws,
                      (unsigned*)a.tickets, a.M, a.K, a.N, a.SKG, a.full, a.out_scale, sp, a.xscale,
                      (unsigned long long*)a.clk,
@@ -472,24 +443,17 @@ void launch_gemv(const r4d_gemv_args& a) {
 
 template <int KB, int MT, int NPW, int SK>
 void launch_gemv_a(const r4d_gemv_args& a) {
-  const int ktw = a.K / 16 / a.SKG;
-  const size_t abytes = gemv_ktl_pad(SK, ktw) * a.M * 32;
   if (a.xf) {
-    if (abytes > kXfAldsMax) r4d::fail("trellis_gemv_xf", "the A slice does not fit LDS: raise SKG");
-    if (a.xf == 2) launch_gemv<KB, MT, NPW, SK, true, 2>(a);
-    else launch_gemv<KB, MT, NPW, SK, true, 1>(a);
+    if (gemv_ktl_pad(SK, a.K / 16 / a.SKG) * a.M * 32 > kXfAldsMax)
+      r4d::fail("trellis_gemv_xf", "the A slice does not fit LDS: raise SKG");
+    if (a.xf == 2) launch_gemv<KB, MT, NPW, SK, 2>(a);
+    else launch_gemv<KB, MT, NPW, SK, 1>(a);
   } else if constexpr (MT == 1) {
     if (a.wsc) {
-      if constexpr (KB == 4 || KB == 5) {
-        if (abytes <= kAldsMax) launch_gemv<KB, MT, NPW, SK, true, 0, true>(a);
-        else launch_gemv<KB, MT, NPW, SK, false, 0, true>(a);
-      } else {
-        r4d::fail("gemm_trellis_nt_m64_wq", "KB must be 4 or 5");
-      }
-    } else if (abytes <= kAldsMax) {
-      launch_gemv<KB, MT, NPW, SK, true, 0>(a);
+      if constexpr (KB == 4 || KB == 5) launch_gemv<KB, MT, NPW, SK, 0, true>(a);
+      else r4d::fail("gemm_trellis_nt_m64_wq", "KB must be 4 or 5");
     } else {
-      launch_gemv<KB, MT, NPW, SK, false, 0>(a);
+      launch_gemv<KB, MT, NPW, SK, 0>(a);
     }
   }
 }
@@ -505,11 +469,14 @@ void launch_gemv_np(const r4d_gemv_args& a, const GemvForm& f) {
   else launch_gemv_a<KB, MT, 2, 4>(a);
 }
 
-// More than one row tile runs here only with the fused transform (A staged whole); trellis_mid.hip has the other forms.
+// Here A's slice is staged whole: more than one row tile, or a slice past kAldsMax, runs here only with the fused transform,
+// and in trellis_mid.hip, which stages it in chunks, otherwise (16 rows, the slice past the limit, us when each wave read
+// its fragments from L2 instead -> now: 5120 x 34816 48.8 -> 41.7, 17408 x 5120 29.1 -> 26.6, KB 5 5120 x 16384 27.6 -> 22.1).
 template <int KB>
 void launch_gemv_kb(const r4d_gemv_args& a, const char* entry) {
   const GemvForm f = gemv_form(a.M, a.N, a.SKG, a.ws != 0 && a.tickets != 0, a.sk1 != 0, a.xf != 0);
-  if (f.MT > 1 && !a.xf) r4d::gemv_mid(a, f.SK == 1, entry);
+  const bool whole = f.MT == 1 && gemv_ktl_pad(f.SK, a.K / 16 / a.SKG) * a.M * 32 <= kAldsMax;
+  if (!a.xf && !whole) r4d::gemv_mid(a, f.SK == 1, entry);
   else if (f.MT <= 1) launch_gemv_np<KB, 1>(a, f);
   else if (f.MT <= 2) launch_gemv_np<KB, 2>(a, f);
   else launch_gemv_np<KB, 4>(a, f);
@@ -670,7 +637,7 @@ const char* r4dx_trellis_gemv_xf_check(int M, int K, int N, int n_split, int KB,
   else {
     const GemvForm f = gemv_form(M, N, SKG, have_ws != 0, false, true);
     if (gemv_ktl_pad(f.SK, K / 16 / SKG) * M * 32 > kXfAldsMax) e = "the A slice does not fit LDS: raise SKG";
-    else if (gemv_form_lds(M, K, N, SKG, have_ws != 0, false, true) > 160 * 1024)
+    else if (gemv_xf_lds(M, K, N, SKG, have_ws != 0) > 160 * 1024)
       e = "the A slice, the split partials and the finish buffers exceed 160 KiB of LDS: lower M or raise SKG";
   }
   return r4d::check_result(e);

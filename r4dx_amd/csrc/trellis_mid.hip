@@ -1,5 +1,6 @@
 // trellis_mid.hip -- the trellis linear for 17..64 rows on gfx950 (r4d_gemm_trellis_nt_m64 and its _raw, _wq, _parts and
-// no-allocation forms above 16 rows): the batch, and the tail of a prompt.
+// no-allocation forms above 16 rows): the batch, and the tail of a prompt. Also up to 16 rows where a K slice of A does not
+// fit the LDS whole (trellis_gemv.hip's rule).
 //
 // DESIGN (MI355X): the decode (about 4 VALU lane-ops per weight) bounds this range, as it does for fewer rows; the MFMAs
 // (2 to 4 row tiles) take a quarter to a half of its time. So the decode stays the GEMV's -- each wave decodes one tile pair
@@ -23,8 +24,8 @@
 
 namespace {
 
-// 64-k steps per staged chunk: 12 or 16 KiB of A per buffer and K part at SK = 1, 24 or 32 KiB over the four parts
-__host__ __device__ constexpr int mid_cs(int MT, int SK) { return SK == 1 ? (MT == 2 ? 4 : 2) : (MT == 2 ? 2 : 1); }
+// 64-k steps per staged chunk: 8 to 16 KiB of A per buffer at SK = 1, 16 to 32 KiB over the four parts at SK = 4
+__host__ __device__ constexpr int mid_cs(int MT, int SK) { return SK == 1 ? (MT <= 2 ? 4 : 2) : (MT <= 2 ? 2 : 1); }
 __host__ __device__ constexpr int mid_stage(int MT, int SK) { return SK * mid_cs(MT, SK) * MT * 2048; }
 constexpr int mid_pairs(int SK) { return SK == 1 ? 4 : 2; }
 
@@ -319,7 +320,7 @@ __global__ __launch_bounds__(64 * mid_pairs(SK) * SK, WQ ? 1 : SK == 1 ? 2 : 4) 
         __hip_atomic_store(m2_flag(out.tickets, blockIdx.x), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       continue;
     }
-    tq_finish<MT, NPW, SK>(acc, lds, out, group, pair, ks, ky);
+    tq_finish<MT, NPW, SK, true>(acc, lds, out, group, pair, ks, ky);
   }
 }
 
@@ -343,7 +344,8 @@ void mid_launch(const r4d_gemv_args& a) {
 }
 template <int KB, int SK, bool WQ>
 void mid_launch_mt(const r4d_gemv_args& a) {
-  if (a.M <= 32) mid_launch<KB, 2, SK, WQ>(a);
+  if (a.M <= 16) mid_launch<KB, 1, SK, WQ>(a);
+  else if (a.M <= 32) mid_launch<KB, 2, SK, WQ>(a);
   else if (a.M <= 48) mid_launch<KB, 3, SK, WQ>(a);
   else mid_launch<KB, 4, SK, WQ>(a);
 }

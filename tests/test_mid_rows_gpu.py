@@ -57,6 +57,27 @@ def test_rows_equal_small_batches(M, K, N, KB, skg, sk):
         assert torch.equal(raw[r:r + 16], ref_raw), f"raw rows {r}.."
 
 
+@pytest.mark.parametrize("M,K,KB,skg,sk", [(1, 40960, 4, 1, 0), (5, 20480, 3, 2, 2), (9, 10880, 5, 2, 0), (13, 5120, 4, 1, 2),
+                                           (16, 13952, 4, 4, 4)])
+def test_long_slices_up_to_16_rows(M, K, KB, skg, sk):
+    """A slice of A past what the M <= 16 kernel stages whole goes through the chunked form: each row carries the bits it has
+    alone (one row of the same slice fits, or is itself past the limit at 40960), and the raw sums are those of the decoded
+    weights."""
+    N = 256
+    g = torch.Generator(device="cuda").manual_seed(K)
+    w = torch.randint(-2**31, 2**31, (K * N * KB // 32,), dtype=torch.int32, device="cuda", generator=g)
+    svh = dev(WL.svh_scales(N, 3))
+    a = torch.randn(M, K, device="cuda", generator=g).half()
+    got, raw = _run(a, w, svh, K, N, KB, skg, sk)
+    for r in range(M):
+        one, one_raw = _run(a[r:r + 1].contiguous(), w, svh, K, N, KB, skg, sk)
+        assert torch.equal(got[r:r + 1], one) and torch.equal(raw[r:r + 1], one_raw)
+    q = api.trellis_reconstruct(w, K, N, KB).view(torch.float16).double()
+    ref = a.double() @ q
+    # fp32 sums of K products: error below K 2^-24 of the terms' magnitudes' sum, here within 1e-5 of the rms
+    assert float((raw.view(torch.float32).double() - ref).abs().max()) < 2e-5 * float(ref.pow(2).mean().sqrt())
+
+
 def test_unsplit_without_ws():
     """SKG = 1 with no ws: data-parallel, the bits of the launch that has one."""
     K, N, M = 2560, 128 * 258, 21
