@@ -218,7 +218,9 @@ size_t r4d_gemm_trellis_nt_i8_ws_bytes(int M, int N, int SKG);
  * beyond the last whole round are cut along K (in up to 8 pieces, whatever skg is; the others are summed whole). */
 int    r4d_mi355x_trellis_i8_skg(int K, int N);
 /* r4d.h:514-521: the coarse sibling: SWC [N] (one scale per column over K), SA [256] (per row, from
- * r4d_trellis_i8_quant_act_row), the int32 sum of the slice scaled once by sa[row] * swc[col]. */
+ * r4d_trellis_i8_quant_act_row), the int32 sum of the slice scaled once by sa[row] * swc[col]. The slices are the skg asked
+ * for, or r4d_mi355x_i8_skg(K, N) where that is fewer and they stay within 131072 k: a finer cut hands the pieces of a
+ * slice over as int32 (through the same ws) and changes no bit. */
 size_t r4d_trellis_i8_wscale_col_count(int K, int N);
 void   r4d_trellis_i8_wscale_col(int64_t w, int64_t swc, int K, int N, int KB, int64_t stream);
 void   r4d_trellis_i8_dump_w_col(int64_t w, int64_t swc, int64_t w8, int64_t wp, int K, int N, int KB, int64_t stream);

@@ -40,6 +40,7 @@ MIN_OCCUPANCY = [            # (demangled name prefix, waves per SIMD at least):
     ("tq_m256_kernel<", 2),      # 8 waves of 64, one workgroup per CU (96 KiB of LDS stages)
     ("tq_m256_finish", 4),
     ("ti8_gemm_kernel<", 2),     # 8 waves, one workgroup per CU
+    ("ti8_exact_finish", 4),
     ("w4_kernel<", 4),
     ("am_kernel<", 8),
 ]

@@ -5,7 +5,7 @@
 //
 // C bf16 [256][N] = bf16((FWHT128(sum) * svh) * out_scale) with
 //   per-128: sum = sum_kb float(int32(A8_kb . W8_kb)) * (sa[kb][row] * sw[kb][col])    (fp32, k-block order)
-//   coarse:  sum = float(int32(A8 . W8 over the slice)) * (sa[row] * sw[col])
+//   coarse:  sum = float(int32(A8 . W8 over the slice)) * (sa[row] * sw[col])      (slices: ti8_run)
 // where W8 is the decoded trellis weight Q quantized on the fly: rs = f16(min(1 / s_eff, 60000)) for the
 // table's s_eff = 1 / rs, q = low byte of f16(w * rs + 1536) (one rounding: round(w * rs) lands in the
 // low byte, the f16 spacing at 1536 being 1) -- the reference's rule (r4d_trellis_i8.h:129-151,
@@ -21,7 +21,8 @@
 // halves (element e of half h <-> k = 8 (e >> 2) + 4 h + (e & 3)) quantize, in that order, to exactly the
 // 16 bytes an MFMA lane needs in A8's k order, so nothing is permuted. Unsplit, the FWHT-128 epilogue runs
 // in registers (column bits 0-3 across lanes, 4-6 across column tiles); split K writes fp32 slices to ws
-// and the split finish pass (trellis_m256.hip) adds them in order and runs the same epilogue.
+// and the split finish pass (trellis_m256.hip) adds them in order and runs the same epilogue. Where a coarse launch
+// is cut finer than its scaled slices, the pieces are int32 and ti8_exact_finish adds them exactly.
 #include "r4d_host.h"
 #include "tq_units.h"
 #include "r4d_mi355x.h"
@@ -191,6 +192,7 @@ struct TI8Args {
   // tail split (tail_s > 1, trellis launches with SKG > 1): column groups below tail_f run whole, the others are cut into
   // tail_s pieces of whole 128-k blocks whose sums go to ws [piece][256][128 (N / 128 - tail_f)]
   int tail_f, tail_s;
+  int exact;            // coarse: ws takes the pieces' int32 sums instead of scaled fp32 ones
 };
 constexpr int kStreamG = 256;                   // workgroups of a stream-K launch (one per CU)
 constexpr int kSlot = 256 * 128;                // values per partial piece
@@ -460,6 +462,20 @@ __device__ __forceinline__ void ti8_piece(const TI8Args& p, unsigned char (*bst)
     }
     return;
   } else {
+    if constexpr (SC == kSCoarse && !DENSE) {
+      if (p.exact && !whole) {
+        const int nw = N - ws_n0;
+        int* dst = (int*)p.ws + (size_t)ky * 256 * nw + (n0 - ws_n0);
+#pragma unroll
+        for (int ii = 0; ii < 2; ++ii)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int ct = 0; ct < 8; ++ct)
+              dst[(size_t)(32 * wave + 16 * ii + 4 * g + j) * nw + 16 * ct + r16] = iacc[ii][ct][j];
+        return;
+      }
+    }
     float v[2][8][4];
     float swc[8];
 #pragma unroll
@@ -593,6 +609,53 @@ __global__ __launch_bounds__(256) void ti8_finish_kernel(const void* __restrict_
   }
 }
 
+// The second pass of a coarse launch cut finer than its scaled slices: ws holds P int32 pieces [P][256][nw] of the columns
+// from n_ws on, P <= 8. `per` consecutive pieces make one slice: added as integers, so its sum is the uncut slice's, then
+// scaled once by sa[row] * sw[col]; the slices are added in order (one slice: it is the sum). FWHT-128, svh, out_scale and
+// the bf16 rounding as in the prefill's finish, whose layout this has: 16 lanes per (row, column group), 8 adjacent columns
+// per lane, every piece requested before any is added (latency-bound: 256 x 2048 in 8 pieces 4.9 us, the fp32 finish of as
+// many 4.8).
+__global__ __launch_bounds__(256) void ti8_exact_finish(TI8Args p, int nw, int n_ws, int P, int per) {
+  const int lane = threadIdx.x & 63;
+  const int r = blockIdx.y * 16 + (threadIdx.x >> 4), wc = blockIdx.x * 128 + 8 * (lane & 15), col = n_ws + wc;
+  const size_t sy = (size_t)256 * nw;
+  const int* src = (const int*)p.ws + (size_t)r * nw + wc;
+  typedef int i4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+  r4i4 t[8][2];
+#pragma unroll
+  for (int y = 0; y < 8; ++y)
+    if (y < P) {
+      t[y][0] = *(const i4_a4*)(src + y * sy);
+      t[y][1] = *(const i4_a4*)(src + y * sy + 4);
+    }
+  float sv[8], sc[8];
+  r4_load_f32<8>(p.svh + col, sv);
+  r4_load_f32<8>(p.sw + col, sc);
+  const float sa = (p.a8[1] != nullptr && n_ws + (int)blockIdx.x * 128 >= p.n_split ? p.sa[1] : p.sa[0])[r];
+  int acc[8] = {0, 0, 0, 0, 0, 0, 0, 0}, left = per;
+  float v[8];
+#pragma unroll
+  for (int y = 0; y < 8; ++y)
+    if (y < P) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] += t[y][e >> 2][e & 3];
+      if (--left == 0) {   // a slice is complete
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float x = (float)acc[e] * (sa * sc[e]);
+          v[e] = per == P ? x : (y < per ? 0.f : v[e]) + x;
+          acc[e] = 0;
+        }
+        left = per;
+      }
+    }
+  r4_fwht128_rows<8>(v, lane);
+  unsigned h[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) h[e] = r4_bf16_rn_sel((v[e] * sv[e]) * p.out_scale);
+  r4_store_u16<8>((unsigned short*)p.c + (size_t)r * p.N + col, h);
+}
+
 std::string ti8_check(int M, int K, int N, int n_split, int KB, int skw, int skg) {
   using r4d::str;
   if (M != 256) return "M must be 256";
@@ -630,6 +693,19 @@ TI8Tail ti8_tail(int K, int N, int cus) {
   return t;
 }
 
+// The fewest K slices (of at least 1024 k, a power of two up to 8) that reach 128 workgroups: the dense form's split, and
+// the coarse trellis form's scaled slices.
+int i8_slices(int K, int N) {
+  const int G = N / 128, nkb = K / 128;
+  int best = 1;
+  for (int d = 1; d <= 8; d *= 2) {         // the split counts r4d_gemm_trellis_nt_i8_check allows
+    if (nkb % d || nkb / d < 8) continue;
+    best = d;
+    if ((long long)G * d >= 128) break;
+  }
+  return best;
+}
+
 template <int KB, int SC, int OUT, bool DENSE>
 void ti8_launch(const TI8Args& a, int N, int SKG, hipStream_t st) {
   if (a.G > 0) hipLaunchKernelGGL((ti8_gemm_kernel<KB, SC, OUT, DENSE>), dim3(a.G), dim3(512), 0, st, a);
@@ -662,7 +738,13 @@ void ti8_run(bool p128, int64_t a8_0, int64_t sa_0, int64_t a8_1, int64_t sa_1, 
   a.N = N;
   a.SKG = skg;
   a.out_scale = out_scale;
-  if (skg > 1) {
+  // The coarse form's sum is a matter of (K, N, skg) only: `slices` scaled sums, each an exact int32 one, however the grid
+  // cuts them -- so a cut for the chip's sake (skg above i8_slices, the tail's pieces) changes no bit. A slice past 2^17 k
+  // could leave int32 (127^2 per k): then the slices are the skg asked for.
+  int slices = skg;
+  if (!p128 && i8_slices(K, N) < skg && K / i8_slices(K, N) <= (1 << 17)) slices = i8_slices(K, N);
+  a.exact = slices < skg;
+  if (skg > 1 && (p128 || slices == 1)) {
     const TI8Tail t = ti8_tail(K, N, r4_cus());
     a.tail_f = t.f;
     a.tail_s = t.s;
@@ -675,7 +757,10 @@ void ti8_run(bool p128, int64_t a8_0, int64_t sa_0, int64_t a8_1, int64_t sa_1, 
     if (p128) ti8_launch<5, kSBlk, kOutBf16, false>(a, N, skg, st);
     else ti8_launch<5, kSCoarse, kOutBf16, false>(a, N, skg, st);
   }
-  if (a.tail_s > 1)
+  if (a.exact) {
+    const int P = a.tail_s > 1 ? a.tail_s : skg, n_ws = a.tail_s > 1 ? 128 * a.tail_f : 0;
+    hipLaunchKernelGGL(ti8_exact_finish, dim3((N - n_ws) / 128, 16), dim3(256), 0, st, a, N - n_ws, n_ws, P, P / slices);
+  } else if (a.tail_s > 1)
     r4d::launch_split_finish(a.ws, a.svh + 128 * a.tail_f, (unsigned short*)a.c + 128 * a.tail_f, M, N - 128 * a.tail_f,
                              a.tail_s, 1, out_scale, st, N);
   else if (skg > 1)
@@ -802,15 +887,17 @@ void r4d_gemm_i8_dense_raw(int64_t a8, int64_t w8, int64_t c, int64_t ws, int64_
 // partials 2 us and 0.045 us per workgroup-slice. Measured, SKG 1 / 2 / 4 (us): per-128 5120 x 16384 90.9 / 58.6 / 67.4,
 // 5120 x 8192 87.1 / 50.3 / 35.7; coarse 5120 x 17408 65.7 / 74.7 / 72.8, 5120 x 10240 64.3 / 40.6 / 47.3, 17408 x 5120
 // 194 / 103 / 59.8, 4096 x 2048 55.3 / 31.3 / 21.2 (SKG 8: 16.7). Above the CUs' number of groups SKG 2 names the tail split
-// (ti8_tail).
+// (ti8_tail). Never fewer than i8_slices, which the coarse form's scaled slices then are (ti8_run).
 int r4d_mi355x_trellis_i8_skg(int K, int N) {
   const int G = N / 128, nkb = K / 128;
   if (G <= 0 || nkb <= 0) return 1;
   const int cus = r4_cus();
   const TI8Tail t = ti8_tail(K, N, cus);
-  int best = 1;
+  int least = i8_slices(K, N);
+  while (least > 1 && nkb % (2 * least)) least /= 2;
+  int best = least;
   double best_cost = 1e30;
-  for (int d = 1; d <= 8; d *= 2) {         // the split counts r4d_gemm_trellis_nt_i8_check allows (with skw 2)
+  for (int d = least; d <= 8; d *= 2) {     // the split counts r4d_gemm_trellis_nt_i8_check allows (with skw 2)
     if (nkb % (2 * d) && d > 1) continue;
     const long long units = (long long)G * d;
     const int steps = 2 * nkb / d;
@@ -827,18 +914,9 @@ int r4d_mi355x_trellis_i8_skg(int K, int N) {
   return best;
 }
 
-// This build's K split for the dense int8 GEMM: the fewest slices (of at least 1024 k) that reach 128
-// workgroups -- the split that measured fastest at both config-4 shapes (1 at 5120 x 17408, 4 at 17408 x 5120).
-int r4d_mi355x_i8_skg(int K, int N) {
-  const int G = N / 128, nkb = K / 128;
-  int best = 1;
-  for (int d = 1; d <= 8; d *= 2) {         // the split counts r4d_gemm_trellis_nt_i8_check allows
-    if (nkb % d || nkb / d < 8) continue;
-    best = d;
-    if ((long long)G * d >= 128) break;
-  }
-  return best;
-}
+// This build's K split for the dense int8 GEMM: i8_slices, the split that measured fastest at 5120 x 17408 (1) and
+// 17408 x 5120 (4).
+int r4d_mi355x_i8_skg(int K, int N) { return i8_slices(K, N); }
 
 // This build's launch form for the dense int8 GEMM by scale mode: the per-128 modes run stream-K (SKG = 0; measured
 // 8-11 % faster than the best split at both config-4 shapes), row / column scales the split above.
