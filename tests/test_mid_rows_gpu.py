@@ -3,8 +3,8 @@ the sizes where its staging, its row tiles and its balanced form can go wrong. E
 gives it in a batch whose slice of A stays within 48 KiB -- the kernel that stages A whole, which shares neither the chunks nor
 the cuts -- in both summation orders, at every rate, for slices whose last step is not whole, parts that are empty or shorter
 than the others, two input parts and more than 8 slices. The balanced form (cut units) at every number of row tiles and every
-rate, at one slice and at two; unsplit, it must also match the launch without ws and tickets, which cuts nothing. Every launch
-leaves its tickets zero."""
+rate, at one slice and at two; unsplit, it must also match the launch without ws and tickets, which cuts nothing, and stay
+inside ws_bytes and tickets_bytes. Every launch leaves its tickets zero."""
 import numpy as np
 import pytest
 
@@ -16,6 +16,7 @@ if not torch.cuda.is_available():
     pytest.skip("no GPU", allow_module_level=True)
 
 from r4dx_amd import api  # noqa: E402
+from r4dx_amd.loader import lib  # noqa: E402
 from gpu_util import banner, dev  # noqa: E402
 
 CASES = [   # (M, K, N, KB, SKG, sk)
@@ -79,6 +80,29 @@ def test_rows_equal_small_batches(M, K, N, KB, skg, sk):
         bare = api.trellis_gemm_m64(a, w, svh, K, N, KB, skg=1, a1=a1, n_split=n_split, out_scale=0.1, sk=sk)
         same = torch.equal(bare.view(torch.int16), got)
         assert same
+
+
+@pytest.mark.parametrize("M,KB", [(64, 4), (29, 5), (12, 3)])
+def test_unsplit_stays_inside_its_workspace(M, KB):
+    """SKG 1 in the SK 1 / 2 order with ws and tickets, cut units or not: nothing outside ws_bytes(M, N, 1) and
+    tickets_bytes(N) is written, the tickets end at zero."""
+    L, K = lib(), 2560
+    for N in (_cols(-7, 1), 512):
+        banner("unsplit workspace", M, K, N, KB)
+        g = torch.Generator(device="cuda").manual_seed(N)
+        w = torch.randint(-2**31, 2**31, (K * N * KB // 32,), dtype=torch.int32, device="cuda", generator=g)
+        a = torch.randn(M, K, device="cuda", generator=g).half()
+        nw, nt = L.r4d_gemm_trellis_nt_m64_ws_bytes(M, N, 1) // 4, L.r4d_gemm_trellis_nt_m64_tickets_bytes(N) // 4
+        ws = torch.full((nw + 8192,), -1, dtype=torch.int32, device="cuda")
+        tk = torch.full((nt + 8192,), 7, dtype=torch.int32, device="cuda")
+        tk[4096:4096 + nt] = 0
+        out = api.trellis_gemm_m64(a, w, dev(WL.svh_scales(N, 3)), K, N, KB, skg=1, ws=ws[4096:4096 + nw],
+                                   tickets=tk[4096:4096 + nt], sk=2)
+        torch.cuda.synchronize()
+        assert bool(torch.isfinite(out.float()).all())
+        assert int((ws[:4096] != -1).sum()) == 0 and int((ws[4096 + nw:] != -1).sum()) == 0
+        assert int((tk[:4096] != 7).sum()) == 0 and int((tk[4096 + nt:] != 7).sum()) == 0
+        assert int(tk[4096:4096 + nt].abs().sum()) == 0
 
 
 @pytest.mark.parametrize("M,K,KB,skg,sk", [(1, 40960, 4, 1, 0), (5, 20480, 3, 2, 2), (9, 10880, 5, 2, 0), (13, 5120, 4, 1, 2),
