@@ -217,8 +217,10 @@ void r4d_gemm_trellis_nt_i8(int64_t a8_0, int64_t sa_0, int64_t a8_1, int64_t sa
 const char* r4d_gemm_trellis_nt_i8_check(int M, int K, int N, int n_split, int KB, int skw, int skg);
 size_t r4d_gemm_trellis_nt_i8_ws_bytes(int M, int N, int SKG);
 /* No reference counterpart (the reference reads gemm_tuning_table_trellis_i8*.inc): this build's skg of the two trellis
- * int8 GEMMs for a shape. With skg > 1 and more column groups than compute units, not a multiple of them, only the groups
- * beyond the last whole round are cut along K (in up to 8 pieces, whatever skg is; the others are summed whole). */
+ * int8 GEMMs for a shape. With skg > 1 and more column groups than compute units, the groups beyond the last whole round
+ * at most half the compute units, only those are cut along K (in up to 8 pieces, whatever skg is; the others are summed
+ * whole); with a larger remainder, or none, every group is cut in skg slices. The per-128 form's fp32 sums are in that order,
+ * so above the compute units' number of groups their last bits depend on it (the coarse form's do not: below). */
 int    r4d_mi355x_trellis_i8_skg(int K, int N);
 /* r4d.h:514-521: the coarse sibling: SWC [N] (one scale per column over K), SA [256] (per row, from
  * r4d_trellis_i8_quant_act_row), the int32 sum of the slice scaled once by sa[row] * swc[col]. The slices are the skg asked
