@@ -56,7 +56,7 @@ __device__ __forceinline__ M2Seg m2_seg(const M2Share& sh, int si, int nst) {
 }
 
 // The reader's side of a cut unit: one thread waits (bounded) for the previous workgroup's flag and clears it for the next
-// launch. Returns whether the wait ran out. `word` is an LDS word free for this; the workgroup meets three barriers.
+// launch. Returns whether the wait ran out. `word` is an LDS word free for this; the workgroup meets two barriers.
 __device__ __forceinline__ bool r4_wait_published(unsigned* flags, int* word) {
   if (threadIdx.x == 0) {
     unsigned* f = m2_flag(flags, blockIdx.x - 1);

@@ -68,9 +68,8 @@ __global__ __launch_bounds__(64 * kM2Waves, 1) void tq_m256_kernel(
 
   const M2Share sh = m2_share(N, SKG, nst, P);
 
-  // The segment preamble both roles run (the same barriers): segment geometry, then, for a continuation, one thread
-  // waits for the previous workgroup's flag (and clears it for the next launch) and tells the workgroup whether it
-  // came in time.
+  // The segment preamble both roles run (the same barriers): segment geometry, then, for a continuation, the wait for
+  // the previous workgroup's flag.
 #define M2_SEGMENT_BEGIN                                                                                   \
     const M2Seg sg = m2_seg(sh, si, nst);                                                                  \
     int Kv = K, Nv = N;                                                                                    \
@@ -83,21 +82,7 @@ __global__ __launch_bounds__(64 * kM2Waves, 1) void tq_m256_kernel(
     const unsigned short* __restrict__ A = r4_part_a(ap, n0);                                              \
     __syncthreads();                                                                                       \
     bool poisoned = false;                                                                                 \
-    if (kind == kSegContinue) {                                                                            \
-      if (threadIdx.x == 0) {                                                                              \
-        unsigned* f = m2_flag(flags, blockIdx.x - 1);                                                        \
-        int spin = 0;                                                                                      \
-        while (__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u && spin < (1 << 24)) { \
-          __builtin_amdgcn_s_sleep(8);                                                                     \
-          ++spin;                                                                                          \
-        }                                                                                                  \
-        __hip_atomic_store(f, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);                             \
-        *(volatile int*)lds = spin < (1 << 24) ? 0 : 1;                                                    \
-      }                                                                                                    \
-      __syncthreads();                                                                                     \
-      poisoned = *(volatile int*)lds != 0;                                                                 \
-      __syncthreads();                                                                                     \
-    }                                                                                                      \
+    if (kind == kSegContinue) poisoned = r4_wait_published(flags, (int*)lds);                              \
     (void)poisoned; (void)A; (void)Kv; (void)Nv; (void)kt0;
 
   if (wave >= 4) {
@@ -496,9 +481,10 @@ std::string m256_check(int M, int K, int N, int n_split, int KB, int SKG) {
   if (KB != 3 && KB != 4 && KB != 5) return "KB " + str(KB) + " is not instantiated (3, 4, 5)";
   if (SKG < 1 || SKG > 64 || (K / 16) % (4 * SKG)) return "SKG must be 1..64 with (K/16) divisible by 4 SKG";
   if (n_split < 0 || n_split > N || n_split % 128) return "n_split must be in 0..N and a multiple of 128";
-  // the kernel's stores and the split finish address one slice, and all SKG slices, with 32-bit buffer offsets
+  // one bound for every split entry's ws, set by the M <= 64 kernel's 32-bit offsets over all its slices; here a slice's
+  // stores alone have them (the finish has 64-bit ones)
   if ((long long)SKG * M * N * 4 > (1LL << 31))
-    return "the fp32 slices SKG * M * N * 4 bytes must fit 2 GiB (32-bit offsets of the split finish): lower SKG";
+    return "the fp32 slices SKG * M * N * 4 bytes must fit 2 GiB: lower SKG";
   return "";
 }
 
