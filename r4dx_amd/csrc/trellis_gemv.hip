@@ -464,9 +464,11 @@ void launch_gemv_a(const r4d_gemv_args& a) {
 // and fewer workgroups take fewer tickets on the group's counter).
 template <int KB, int MT>
 void launch_gemv_np(const r4d_gemv_args& a, const GemvForm& f) {
-  if (f.SK == 1) launch_gemv_a<KB, MT, 4, 1>(a);
-  else if (f.NPW == 1) launch_gemv_a<KB, MT, 1, 4>(a);
-  else launch_gemv_a<KB, MT, 2, 4>(a);
+  if (f.SK == 1) return launch_gemv_a<KB, MT, 4, 1>(a);
+  if constexpr (MT == 1) {                     // one pair per workgroup: M = 1 only (gemv_form)
+    if (f.NPW == 1) return launch_gemv_a<KB, MT, 1, 4>(a);
+  }
+  launch_gemv_a<KB, MT, 2, 4>(a);
 }
 
 // Here A's slice is staged whole: more than one row tile, or a slice past kAldsMax, runs here only with the fused transform,
