@@ -30,13 +30,17 @@ EXTRA = {"trellis_i8.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=true"]}
 # (-Rpass-analysis=kernel-resource-usage) must show no scratch and no spills, and each kernel family keeps at least
 # the occupancy (waves per SIMD) its design and measurements assume. The report goes to _build/resources.json.
 REMARK = "-Rpass-analysis=kernel-resource-usage"
+# the chunked kernel by (SK, fake-quant): waves per SIMD at 1..4 row tiles, at every rate
+MID_OCCUPANCY = {(1, "false"): (3, 2, 2, 2), (4, "false"): (4, 4, 4, 4), (1, "true"): (2, 2, 1, 1), (4, "true"): (3, 3, 3, 2)}
 MIN_OCCUPANCY = [            # (demangled name prefix, waves per SIMD at least): every matching prefix applies
-    ("tq_gemv_kernel<4, 1, 1, 4,", 5),   # the decode GEMV at M = 1 (KB 4): VALU latency hiding
-    ("tq_gemv_kernel<4, 1, 2, 4, 0, false>", 6),   # ... at M = 2..16
-    ("tq_gemv_kernel<5, 1, 1, 4, 0, false>", 5),
+    ("tq_gemv_kernel<4, 1, 1, 4,", 5),   # the decode GEMV at M = 1, fake-quant included: VALU latency hiding
+    ("tq_gemv_kernel<4, 1, 1, 4, 0, false>", 7), ("tq_gemv_kernel<5, 1, 1, 4, 0, false>", 7),
+    ("tq_gemv_kernel<4, 1, 2, 4, 0, false>", 7), ("tq_gemv_kernel<5, 1, 2, 4, 0, false>", 7),   # ... at M = 2..16
+    ("tq_gemv_kernel<3, 1, 1, 4, 0, false>", 8), ("tq_gemv_kernel<3, 1, 2, 4, 0, false>", 8),
+    *[(f"tq_gemv_kernel<{kb}, 1, {npw}, 4, {xf}, false>", 6) for kb in (3, 4, 5) for npw in (1, 2) for xf in (1, 2)],   # fused
     ("tq_gemv_kernel<", 2),
-    ("tq_mid_kernel<", 1),       # 17..64 rows; the fake-quant forms take what they need
-    ("tq_mid_kernel<4, 2, 1, false>", 2), ("tq_mid_kernel<4, 2, 4, false>", 4), ("tq_mid_kernel<4, 4, 4, false>", 4),
+    *[(f"tq_mid_kernel<{kb}, {i + 1}, {sk}, {wq}>", n) for kb in (3, 4, 5) for (sk, wq), ns in MID_OCCUPANCY.items()
+      for i, n in enumerate(ns)],
     ("tq_m256_kernel<", 2),      # 8 waves of 64, one workgroup per CU (96 KiB of LDS stages)
     ("tq_m256_finish", 4),
     ("ti8_gemm_kernel<", 2),     # 8 waves, one workgroup per CU
@@ -45,9 +49,12 @@ MIN_OCCUPANCY = [            # (demangled name prefix, waves per SIMD at least):
     ("am_kernel<", 8),
 ]
 # Kernels allowed a few SGPR spills (at most this many; they go to VGPR lanes by v_writelane, never to memory, and the
-# gate still requires no scratch and no VGPR spill): the prefill GEMM and the 17..64-row kernel keep their launch arguments
-# and the per-segment geometry of the balanced form in scalars across the whole kernel, outside the step loop.
-SGPR_LANE_SPILLS = [("tq_m256_kernel<", 16), ("tq_mid_kernel<", 48)]
+# gate still requires no scratch and no VGPR spill): the prefill GEMM and the chunked kernel's balanced order (SK 1) keep
+# their launch arguments and the per-segment geometry in scalars across the whole kernel, outside the step loop. The limits
+# are what the kernels have today (the fake-quant forms carry two more arguments).
+SGPR_LANE_SPILLS = [("tq_m256_kernel<", 11),
+                    *[(f"tq_mid_kernel<{kb}, {mt}, 1, {wq}>", n) for kb in (3, 4, 5) for mt in (1, 2, 3, 4)
+                      for wq, n in (("false", 36), ("true", 44))]]
 
 
 def parse_resources(text):

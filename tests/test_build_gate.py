@@ -33,6 +33,21 @@ def test_gate_parses_and_flags():
     assert any("occupancy 4" in b for b in B.gate(recs))
 
 
+def test_every_chunked_form_has_its_own_limits():
+    """No tq_mid_kernel form rests on a family-wide floor: one wave fewer, or one spill more, fails."""
+    for kb in (3, 4, 5):
+        for mt in (1, 2, 3, 4):
+            for sk in (1, 4):
+                for wq in ("false", "true"):
+                    name = f"tq_mid_kernel<{kb}, {mt}, {sk}, {wq}>(R4AParts)"
+                    floors = [n for prefix, n in B.MIN_OCCUPANCY if name.startswith(prefix)]
+                    assert floors, name
+                    spills = [n for prefix, n in B.SGPR_LANE_SPILLS if name.startswith(prefix)]
+                    rec = dict(name=name, mangled=name, Occupancy=max(floors), SGPRsSpill=max(spills or [0]))
+                    assert B.gate([rec]) == []
+                    assert B.gate([dict(rec, Occupancy=max(floors) - 1)]) and B.gate([dict(rec, SGPRsSpill=max(spills or [0]) + 1)])
+
+
 def test_built_library_passes_the_gate():
     path = os.path.join(B.PKG, "_build", "resources.json")
     if not os.path.exists(path):
