@@ -39,6 +39,7 @@ MIN_OCCUPANCY = [            # (demangled name prefix, waves per SIMD at least):
     ("tq_gemv_kernel<3, 1, 1, 4, 0, false>", 8), ("tq_gemv_kernel<3, 1, 2, 4, 0, false>", 8),
     *[(f"tq_gemv_kernel<{kb}, 1, {npw}, 4, {xf}, false>", 6) for kb in (3, 4, 5) for npw in (1, 2) for xf in (1, 2)],   # fused
     ("tq_gemv_kernel<", 2),
+    ("tq_mid_kernel<4, 1, 4, false>", 5), ("tq_mid_kernel<3, 1, 4, false>", 5),
     *[(f"tq_mid_kernel<{kb}, {i + 1}, {sk}, {wq}>", n) for kb in (3, 4, 5) for (sk, wq), ns in MID_OCCUPANCY.items()
       for i, n in enumerate(ns)],
     ("tq_m256_kernel<", 2),      # 8 waves of 64, one workgroup per CU (96 KiB of LDS stages)
