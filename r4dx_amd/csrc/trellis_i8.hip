@@ -559,23 +559,37 @@ template <int KB, int SC, int OUT, bool DENSE>
 __global__ __launch_bounds__(512, 1) void ti8_gemm_kernel(TI8Args p) {
   __shared__ __attribute__((aligned(16))) unsigned char bst[2][4][128][16];   // [stage][k-tile][column slot][16 B]
   __shared__ int flag;
-  if constexpr (!DENSE) {
-    if (p.tail_s > 1) {
-      // the pieces first: a CU that ran one takes a whole group next, and the last round is whole groups only
-      const int pieces = (p.N / 128 - p.tail_f) * p.tail_s, b = blockIdx.x;
-      if (b < pieces) {
-        const int g = b / p.tail_s, y = b - g * p.tail_s, nb = p.K >> 7;
-        const int b0 = (int)((long long)y * nb / p.tail_s), b1 = (int)((long long)(y + 1) * nb / p.tail_s);
-        ti8_piece<KB, SC, OUT, DENSE>(p, bst, &flag, p.tail_f + g, y, 8 * b0, 2 * (b1 - b0), -1, 128 * p.tail_f);
-      } else {
-        ti8_piece<KB, SC, OUT, DENSE>(p, bst, &flag, b - pieces, 0, 0, p.K >> 6, -1, 0, true);
-      }
-      return;
-    }
-  }
   if (!DENSE || p.G == 0) {
     const int ktw = (p.K >> 4) / p.SKG;
-    ti8_piece<KB, SC, OUT, DENSE>(p, bst, &flag, blockIdx.x, blockIdx.y, blockIdx.y * ktw, ktw >> 2, -1);
+    int group = blockIdx.x, ky = blockIdx.y, kt0 = ky * ktw, nst = ktw >> 2, ws_n0 = 0;
+    bool whole = false;
+    // One copy of the body for all three launch roles, or one copy each: which schedules better is the compiler's
+    // register allocation, measured (us, one / three): KB 5 per-128 5120 x 17408 94.5 / 97.4 (94.9 without the tail split's
+    // roles), 17408 x 5120 84.3 / 86.7; KB 4 per-128 92.6 / 90.4 and 82.7 / 80.8; KB 5 coarse 70.7 / 68.9, KB 4 66.4 / 66.0.
+    constexpr bool kOneBody = KB == 5 && SC == kSBlk;
+    if constexpr (!DENSE) {
+      if (p.tail_s > 1) {
+        // the pieces first: a CU that ran one takes a whole group next, and the last round is whole groups only
+        const int pieces = (p.N / 128 - p.tail_f) * p.tail_s, b = blockIdx.x, nb = p.K >> 7;
+        if (b < pieces) {
+          const int g = b / p.tail_s, y = b - g * p.tail_s;
+          const int b0 = (int)((long long)y * nb / p.tail_s), b1 = (int)((long long)(y + 1) * nb / p.tail_s);
+          group = p.tail_f + g;
+          ky = y;
+          kt0 = 8 * b0;
+          nst = 2 * (b1 - b0);
+          ws_n0 = 128 * p.tail_f;
+          if constexpr (!kOneBody) return ti8_piece<KB, SC, OUT, DENSE>(p, bst, &flag, group, ky, kt0, nst, -1, ws_n0);
+        } else {
+          group = b - pieces;
+          kt0 = 0;
+          nst = 2 * nb;
+          whole = true;
+          if constexpr (!kOneBody) return ti8_piece<KB, SC, OUT, DENSE>(p, bst, &flag, group, 0, 0, nst, -1, 0, true);
+        }
+      }
+    }
+    ti8_piece<KB, SC, OUT, DENSE>(p, bst, &flag, group, ky, kt0, nst, -1, kOneBody ? ws_n0 : 0, kOneBody && whole);
     return;
   }
   // stream-K: this workgroup's units [u0, u1), a unit = (group, 128-k block) = 2 steps
