@@ -46,7 +46,7 @@ MIN_OCCUPANCY = [            # (demangled name prefix, waves per SIMD at least):
     ("tq_m256_finish", 4),
     ("ti8_gemm_kernel<", 2),     # 8 waves, one workgroup per CU
     ("ti8_exact_finish", 4),
-    ("w4_kernel<", 4),
+    ("w4_kernel<", 4), ("w4_kernel<32, 32,", 6), ("w4_kernel<64, 32,", 6),
     ("am_kernel<", 8),
 ]
 # Kernels allowed a few SGPR spills (at most this many; they go to VGPR lanes by v_writelane, never to memory, and the

@@ -24,8 +24,9 @@
 // k +8, +10, +9, +11 ("V"). A 64-k block is four MFMAs of eight elements per lane: U of dwords (0, 1), U of (2, 3), V of
 // (0, 1), V of (2, 3) -- each inside one group of 32; a group's MFMAs form one chain, whose sum takes the group's scale in
 // one fma per output. (With 16 (q - z) for the high nibbles a group had two chains and two fmas per output: above 8 rows
-// those 64 fmas per block at two row tiles weighed more than the MFMAs: 24 rows G = 32 216 -> 197 us, 64 rows 390 -> 366.) The A fragment of an MFMA is two runs of four k in
-// that order, staged in LDS with one row of zeros per (block, MFMA, k-half) for the lanes whose row is absent.
+// those 64 fmas per block at two row tiles weighed more than the MFMAs: 24 rows G = 32 214 -> 197 us, 64 rows
+// 385 -> 354.) The A fragment of an MFMA is two runs of four k in that order, staged in LDS with one row of zeros per
+// (block, MFMA, k-half) for the lanes whose row is absent.
 //
 // Two MFMA forms. M <= 8: v_mfma_f32_16x16x32_f16 with rows (2 m + tile): lane (n, kq) holds the B data
 // of tile kq & 1, k-half kq >> 1, and A row rho is nonzero only where rho & 1 == kq & 1, so output row
@@ -248,7 +249,8 @@ __device__ __forceinline__ void w4_store_argmax(const Acc (&acc)[SMALL ? 1 : MT]
 
 // MR: the form's rows, the next of {1, 2, 4, 8, 32, 64} from M on. SMALL (MR <= 8): the 16x16x32 form, whose MR + 1 staged rows
 // have a constant stride, so fragment addresses are one register plus immediates and the staging divides nothing (with M +
-// 1 rows, G = 32, 1 / 4 / 8 rows: 144 / 161 / 156 -> 135 / 148 / 151 us at 5120 x 248320 with argmax; at G = 64 up to 2 %).
+// 1 rows, G = 32, 1 / 2 / 4 / 8 rows: 140 / 138 / 139 / 146 -> 137 / 132 / 136 / 145 us at 5120 x 248320 with argmax; at G = 64 up
+// to 2 %).
 // Above that MT row tiles of 32 in the 32x32x16 form with M + 1 staged rows (padded rows shorten the chunks: 2 to 5 % slower).
 // AM (with OUTF): the fused per-row argmax of the logits (AmFused).
 template <int G, int MR, bool OUTF, bool AM>
@@ -384,6 +386,18 @@ __global__ __launch_bounds__(64 * kWaves, MR <= 8 ? (G == 32 ? 8 : 6) : 1) void 
       __device__ unsigned operator[](int i) const { return p[i]; }
     };
     const struct { SzView sz; } s{SzView{COOP ? szl : s0.sz}};
+    // One row tile of 32, G = 64: the chain's first fragments are requested before the dequant. With one chain the compiler
+    // asked for each only as the MFMA before it ran, so three LDS round trips of a block stood open where few waves share a
+    // SIMD (16 rows, 5120 x 16384, two chains / one / one with early reads: fused argmax 47.0 / 47.4 / 44.7 us, f32 40.8 / 42.4
+    // / 41.0). As many as leave 6 waves per SIMD, which the large vocabularies need (fused 5120 x 248320, 24 rows:
+    // none 180 us, 2 early 177, 4 early at 5 waves 184); at G = 32, chains of two MFMAs, early reads lost up to 3 % there.
+    constexpr int kEarlyA = MR == 32 && G == 64 ? (AM ? 2 : 1) : 0;
+    r4h8 af[kEarlyA ? kEarlyA : 1];
+    if constexpr (kEarlyA > 0) {
+#pragma unroll
+      for (int u = 0; u < kEarlyA; ++u) af[u] = afrag(0, kbl, (u & 1) * 2 + (u >> 1));   // the chain's order
+      __builtin_amdgcn_sched_barrier(0x47F);   // LDS reads do not cross
+    }
     unsigned nz[4], nzv[4];
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
@@ -408,7 +422,7 @@ __global__ __launch_bounds__(64 * kWaves, MR <= 8 ? (G == 32 ? 8 : 6) : 1) void 
           const int c = G == 64 ? (u & 1) * 2 + (u >> 1) : g + 2 * u, ch = u & (kCh - 1);
           const Acc t0 = u < kCh ? Acc{} : t[ch];
           if constexpr (SMALL) t[ch] = __builtin_amdgcn_mfma_f32_16x16x32_f16(afrag(i, kbl, c), w4_bop(bq, c), t0, 0, 0, 0);
-          else t[ch] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afrag(i, kbl, c), w4_bop(bq, c), t0, 0, 0, 0);
+          else t[ch] = __builtin_amdgcn_mfma_f32_32x32x16_f16(u < kEarlyA ? af[u < kEarlyA ? u : 0] : afrag(i, kbl, c), w4_bop(bq, c), t0, 0, 0, 0);
         }
         if constexpr (SMALL) {
           // output rows 4 (lane >> 4) + e = 2 m + t: tile t = e & 1 (rows m >= M have zero A and stay 0)
@@ -449,6 +463,10 @@ __global__ __launch_bounds__(64 * kWaves, MR <= 8 ? (G == 32 ? 8 : 6) : 1) void 
     for (int i = 0; i < kPF; ++i) {
       compute(ring[i], kb - kb_chunk + i);
       load(ring[i], kb + i + kPF);
+      // one step at a time: left to itself the scheduler moved the next steps' loads behind this one's use at G = 64 and
+      // kept half of the ring in flight (5120 x 16384 with f32 logits, 1 / 4 / 8 rows: 26.9 / 29.4 / 32.0 -> 24.8 / 26.0 / 29.0
+      // us; from 65536 columns on the stream bounds it either way)
+      if constexpr (SMALL && G == 64) __builtin_amdgcn_sched_barrier(0);
     }
   }
   if (full < KB64) {
