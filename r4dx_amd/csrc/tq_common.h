@@ -124,11 +124,11 @@ constexpr size_t tq_end_lds(int MT, int NPW, int SK, int M) { return tq_end_lds_
 // A unit's end, after tq_combine. Lane l of wave (pl, ks = 0) holds rows 16 i + 4 (l >> 4) + j of column slot nb = l & 15
 // of fragment cs: true column 32 pair + 16 (nb >> 3) + (nb & 7) + 8 cs.
 //   * SKG = 1, raw: the sums are C.
-//   * SKG = 1 in a workgroup that holds its whole group (NPW = 4): the sums meet in LDS.
+//   * SKG = 1 in a workgroup that holds its whole group (NPW = 4): the sums meet in LDS and are finished from there.
 //   * else the partials go to ws -- above one row tile through LDS, as 16-byte row pieces (the accumulators' own 4-byte
-//     stores cost 3 to 5 us a launch at 49 and 64 rows) -- and the last of the group's SKG 4 / NPW contributors (ticket) sums the slices: run p
-//     (0..7) is 0.f + slices p, p + 8, ... in order, then the runs in order 0..7 (an absent slice adds +0.f, which changes
-//     nothing) -- the same arithmetic for every element whatever M is. The loads are coherent (sc1) 16-byte buffer loads,
+//     stores cost 3 to 5 us a launch at 49 and 64 rows) -- and the last of the group's SKG 4 / NPW contributors (ticket)
+//     sums the slices: run p (0..7) is 0.f + slices p, p + 8, ... in order, then the runs in order 0..7 (an absent slice
+//     adds +0.f, which changes nothing) -- the same arithmetic for every element whatever M is. The loads are coherent (sc1) 16-byte buffer loads,
 //     every slice of a batch of 8 requested before any is added.
 // Each 32-lane half of a wave then owns one row's 128 sums, 4 adjacent columns per lane, from the slice sum to the
 // store (r4_fwht128_rows): no LDS copy of the slice sums, no stage through the LDS crossbar and one 8-byte store per lane.
@@ -160,13 +160,43 @@ __device__ __forceinline__ void tq_finish(const r4f4 (&acc)[MT][2], unsigned cha
     }
     return;
   }
-  const bool in_block = NPW == 4 && SK == 1 && SKG == 1;   // the workgroup holds its whole group
+  const int c0 = 4 * (lane & 31);               // the 4 columns this lane finishes
+  if constexpr (NPW == 4 && SK == 1) {
+    // The workgroup holds its whole group. A path of its own, short and in line with the k loop: run through the split's
+    // code below, with svh asked for behind the barrier, an unsplit launch took 0.2 us more at 1 row, whatever K, and up to
+    // 1.3 us at 64 (128 x 1024, 17 / 64 rows 5.0 / 7.5 -> 4.3 / 6.2 us; 5120 x 34816, 64 rows 68.9 -> 67.9).
+    if (SKG == 1) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int r = 16 * i + 4 * rq + j;
+          if (r < M) {
+            red[r * 128 + gcol0] = acc[i][0][j];
+            red[r * 128 + gcol0 + 8] = acc[i][1][j];
+          }
+        }
+      float sv[4];
+      r4_load_f32<4>(o.svh + n0 + c0, sv);      // in flight over the barrier
+      __syncthreads();
+      for (int r = (int)threadIdx.x >> 5; r < M; r += NT / 32) {
+        float v[4];
+        r4_load_f32<4>(red + r * 128 + c0, v);
+        r4_fwht128_rows<4>(v, lane);
+        unsigned h[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[e] = r4_bf16_rn_sel((v[e] * sv[e]) * o.out_scale);
+        r4_store_u16<4>(Cb + (size_t)r * N + n0 + c0, h);
+      }
+      return;
+    }
+  }
   // the partials pass through LDS and leave as whole 16-byte row pieces (up to 8 rows their few 4-byte stores are as fast)
   const bool staged = MT > 1 || (STAGE && M > 8);
   constexpr int kCols = 32 * NPW;               // the workgroup's columns
   const unsigned sy4 = (unsigned)M * (unsigned)N * 4u;
   const r4_rsrc wsr = r4_make_rsrc(o.ws, (unsigned)SKG * sy4);
-  if (in_block || staged) {
+  if (staged) {
     if constexpr (SK > 1) __syncthreads();      // the part accumulators have been read
     const int lcol0 = gcol0 & (kCols - 1);
     if (ks == 0) {
@@ -182,33 +212,28 @@ __device__ __forceinline__ void tq_finish(const r4f4 (&acc)[MT][2], unsigned cha
         }
     }
     __syncthreads();
-  }
-  if (!in_block) {
-    if (staged) {
-      const unsigned base = (unsigned)ky * sy4 + (unsigned)(n0 + (kCols == 128 ? 0 : (pair * 32) & (128 - kCols))) * 4u;
-      for (int it = (int)threadIdx.x; it < M * (kCols / 4); it += NT) {
-        const int r = it / (kCols / 4), cq = it & (kCols / 4 - 1);
-        __builtin_amdgcn_raw_buffer_store_b128(*(const r4u4*)(red + r * kCols + 4 * cq), wsr,
-                                               base + (unsigned)r * (unsigned)N * 4u + 16u * cq, 0, 16);
-      }
-    } else if (ks == 0) {
-      float* wsy = o.ws + (size_t)ky * M * N;
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int r = 16 * i + 4 * rq + j;
-          if (r < M) {
-            r4_store_coherent(&wsy[(size_t)r * N + n0 + gcol0], acc[i][0][j]);
-            r4_store_coherent(&wsy[(size_t)r * N + n0 + gcol0 + 8], acc[i][1][j]);
-          }
-        }
+    const unsigned base = (unsigned)ky * sy4 + (unsigned)(n0 + (kCols == 128 ? 0 : (pair * 32) & (128 - kCols))) * 4u;
+    for (int it = (int)threadIdx.x; it < M * (kCols / 4); it += NT) {
+      const int r = it / (kCols / 4), cq = it & (kCols / 4 - 1);
+      __builtin_amdgcn_raw_buffer_store_b128(*(const r4u4*)(red + r * kCols + 4 * cq), wsr,
+                                             base + (unsigned)r * (unsigned)N * 4u + 16u * cq, 0, 16);
     }
-    if (!r4_ticket_last(&o.tickets[group * R4_TICKET_WORDS], (unsigned)(SKG * (4 / NPW)),
-                        (int*)(lds + tq_end_lds_flag(MT, NPW, SK, M))))
-      return;
+  } else if (ks == 0) {
+    float* wsy = o.ws + (size_t)ky * M * N;
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int r = 16 * i + 4 * rq + j;
+        if (r < M) {
+          r4_store_coherent(&wsy[(size_t)r * N + n0 + gcol0], acc[i][0][j]);
+          r4_store_coherent(&wsy[(size_t)r * N + n0 + gcol0 + 8], acc[i][1][j]);
+        }
+      }
   }
-  const int c0 = 4 * (lane & 31);               // this lane's 4 columns
+  if (!r4_ticket_last(&o.tickets[group * R4_TICKET_WORDS], (unsigned)(SKG * (4 / NPW)),
+                      (int*)(lds + tq_end_lds_flag(MT, NPW, SK, M))))
+    return;
   float sv[4] = {0.f, 0.f, 0.f, 0.f};
   if (full) r4_load_f32<4>(o.svh + n0 + c0, sv);
   // rows per thread and pass, all their slices requested at once (one row at a time, a workgroup at 49 rows made seven
@@ -216,59 +241,50 @@ __device__ __forceinline__ void tq_finish(const r4f4 (&acc)[MT][2], unsigned cha
   constexpr int kU = MT == 1 || (MT == 4 && SK == 4) ? 1 : 2;
   for (int it0 = (int)threadIdx.x; it0 < M * 32; it0 += kU * NT) {
     float v[kU][4];
-    if (in_block) {
+    unsigned off[kU];
 #pragma unroll
-      for (int u = 0; u < kU; ++u) {
-        const r4f4 a = *(const r4f4*)(red + min((it0 + u * NT) >> 5, M - 1) * kCols + (c0 & (kCols - 1)));
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[u][e] = a[e];
-      }
-    } else {
-      unsigned off[kU];
+    for (int u = 0; u < kU; ++u)
+      off[u] = ((unsigned)min((it0 + u * NT) >> 5, M - 1) * (unsigned)N + (unsigned)(n0 + c0)) * 4u;
+    auto slice = [&](int u, unsigned sy) {
+      return __builtin_bit_cast(r4f4, __builtin_amdgcn_raw_buffer_load_b128(wsr, off[u] + sy, 0, 16));
+    };
+    // at most one slice per run (every planned split): branch-free, a slice past SKG reads past the buffer and gives the
+    // +0.f of an empty run (a load under a branch would also keep its registers live around the caller's loop)
+    auto few = [&](auto n) {
+      constexpr int kN = decltype(n)::value;
+      r4f4 t[kU][kN];
 #pragma unroll
       for (int u = 0; u < kU; ++u)
-        off[u] = ((unsigned)min((it0 + u * NT) >> 5, M - 1) * (unsigned)N + (unsigned)(n0 + c0)) * 4u;
-      auto slice = [&](int u, unsigned sy) {
-        return __builtin_bit_cast(r4f4, __builtin_amdgcn_raw_buffer_load_b128(wsr, off[u] + sy, 0, 16));
-      };
-      // at most one slice per run (every planned split): branch-free, a slice past SKG reads past the buffer and gives the
-      // +0.f of an empty run (a load under a branch would also keep its registers live around the caller's loop)
-      auto few = [&](auto n) {
-        constexpr int kN = decltype(n)::value;
-        r4f4 t[kU][kN];
 #pragma unroll
-        for (int u = 0; u < kU; ++u)
+        for (int p = 0; p < kN; ++p) t[u][p] = slice(u, p < SKG ? (unsigned)p * sy4 : 0x80000000u);
 #pragma unroll
-          for (int p = 0; p < kN; ++p) t[u][p] = slice(u, p < SKG ? (unsigned)p * sy4 : 0x80000000u);
+      for (int u = 0; u < kU; ++u)
 #pragma unroll
-        for (int u = 0; u < kU; ++u)
+        for (int e = 0; e < 4; ++e) {
+          v[u][e] = 0.f + t[u][0][e];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            v[u][e] = 0.f + t[u][0][e];
+          for (int p = 1; p < kN; ++p) v[u][e] += 0.f + t[u][p][e];
+          if (kN < 8) v[u][e] += 0.f;
+        }
+    };
+    if (SKG <= 4) {
+      few(std::integral_constant<int, 4>());
+    } else if (SKG <= 8) {
+      few(std::integral_constant<int, 8>());
+    } else {
 #pragma unroll
-            for (int p = 1; p < kN; ++p) v[u][e] += 0.f + t[u][p][e];
-            if (kN < 8) v[u][e] += 0.f;
-          }
-      };
-      if (SKG <= 4) {
-        few(std::integral_constant<int, 4>());
-      } else if (SKG <= 8) {
-        few(std::integral_constant<int, 8>());
-      } else {
-#pragma unroll
-        for (int u = 0; u < kU; ++u) {
+      for (int u = 0; u < kU; ++u) {
 #pragma unroll 1
-          for (int p = 0; p < 8; ++p) {
-            float run[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int p = 0; p < 8; ++p) {
+          float run[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-            for (int y = p; y < SKG; y += 8) {
-              const r4f4 t = slice(u, (unsigned)y * sy4);
+          for (int y = p; y < SKG; y += 8) {
+            const r4f4 t = slice(u, (unsigned)y * sy4);
 #pragma unroll
-              for (int e = 0; e < 4; ++e) run[e] += t[e];
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[u][e] = p == 0 ? run[e] : v[u][e] + run[e];
+            for (int e = 0; e < 4; ++e) run[e] += t[e];
           }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[u][e] = p == 0 ? run[e] : v[u][e] + run[e];
         }
       }
     }
