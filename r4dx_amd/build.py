@@ -37,6 +37,8 @@ MIN_OCCUPANCY = [            # (demangled name prefix, waves per SIMD at least):
     ("tq_gemv_kernel<4, 1, 1, 4, 0, false>", 7), ("tq_gemv_kernel<5, 1, 1, 4, 0, false>", 7),
     ("tq_gemv_kernel<4, 1, 2, 4, 0, false>", 7), ("tq_gemv_kernel<5, 1, 2, 4, 0, false>", 7),   # ... at M = 2..16
     ("tq_gemv_kernel<3, 1, 1, 4, 0, false>", 8), ("tq_gemv_kernel<3, 1, 2, 4, 0, false>", 8),
+    *[(f"tq_gemv_kernel<{kb}, {mt}, {npw}, {sk}, 0, false>", n) for kb in (3, 4, 5)       # 17..64 rows, A staged whole
+      for mt, npw, sk, n in ((2, 4, 1, 3), (2, 2, 4, 5), (4, 4, 1, 2))],
     *[(f"tq_gemv_kernel<{kb}, 1, {npw}, 4, {xf}, false>", 6) for kb in (3, 4, 5) for npw in (1, 2) for xf in (1, 2)],   # fused
     ("tq_gemv_kernel<", 2),
     ("tq_mid_kernel<4, 1, 4, false>", 5), ("tq_mid_kernel<3, 1, 4, false>", 5),

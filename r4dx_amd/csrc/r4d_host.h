@@ -104,6 +104,6 @@ namespace r4d {
 // Checks and launches one trellis GEMV (trellis_gemv.hip); throws std::runtime_error naming `entry` on an illegal
 // launch.
 void gemv_run(r4d_gemv_args& a, const char* entry);
-// The form that stages A in chunks (trellis_mid.hip: 17..64 rows, long slices) of a checked launch; sk1: one wave per tile pair over the whole K slice.
+// The form that stages A in chunks (trellis_mid.hip) of a checked launch; sk1: one wave per tile pair over the whole K slice.
 void gemv_mid(const r4d_gemv_args& a, bool sk1, const char* entry);
 }  // namespace r4d

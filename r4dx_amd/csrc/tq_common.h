@@ -1,6 +1,6 @@
-// tq_common.h -- what the M <= 64 trellis kernels (trellis_gemv.hip: M <= 16 and the fused transform; trellis_mid.hip:
-// M = 17..64) share: the weight words' loads, the K-part combine, the split hand-over with its fixed-order slice sum, and
-// the FWHT-128 epilogue. A linear's bits depend on (K, N, KB, SKG, SK) only, so both kernels run these very sums.
+// tq_common.h -- what the M <= 64 trellis kernels (trellis_gemv.hip: a K slice of A staged whole, and the fused transform;
+// trellis_mid.hip: in chunks) share: the weight words' loads, the K-part combine, the split hand-over with its fixed-order
+// slice sum, and the FWHT-128 epilogue. A linear's bits depend on (K, N, KB, SKG, SK) only, so both kernels run these very sums.
 #pragma once
 #include "r4d_dev.h"
 

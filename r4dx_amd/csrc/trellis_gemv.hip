@@ -1,6 +1,7 @@
-// trellis_gemv.hip -- the trellis linear for M = 1..64 rows on gfx950 (the kernel of M <= 16 and of the fused input
-// transform; trellis_mid.hip has 17..64): r4d_gemm_trellis_nt_m64, its _raw fp32 entry, r4d_trellis_reconstruct_f16 and the ticket helpers (the C ABI of the reference's
-// third_party/libr4d/r4d.h:344-393, kernel semantics of r4d_gemm_trellis_nt_m64.hip:215-503).
+// trellis_gemv.hip -- the trellis linear for M = 1..64 rows on gfx950: r4d_gemm_trellis_nt_m64, its _raw fp32 entry,
+// r4d_trellis_reconstruct_f16 and the ticket helpers (the C ABI of the reference's third_party/libr4d/r4d.h:344-393, kernel
+// semantics of r4d_gemm_trellis_nt_m64.hip:215-503). The kernel here stages a workgroup's K slice of A whole; slices that do
+// not fit, and most of 17..64 rows, are trellis_mid.hip's (launch_gemv_kb has the rule).
 //
 // C[m][n] = bf16((FWHT128(A_p(n) @ Q)[m][n] * svh[n]) * out_scale)   (full), or fp32 A @ Q (_raw).
 //
@@ -448,7 +449,7 @@ void launch_gemv_a(const r4d_gemv_args& a) {
       r4d::fail("trellis_gemv_xf", "the A slice does not fit LDS: raise SKG");
     if (a.xf == 2) launch_gemv<KB, MT, NPW, SK, 2>(a);
     else launch_gemv<KB, MT, NPW, SK, 1>(a);
-  } else if constexpr (MT == 1) {
+  } else if constexpr (MT <= 2 || SK == 1) {
     if (a.wsc) {
       if constexpr (KB == 4 || KB == 5) launch_gemv<KB, MT, NPW, SK, 0, true>(a);
       else r4d::fail("gemm_trellis_nt_m64_wq", "KB must be 4 or 5");
@@ -471,13 +472,18 @@ void launch_gemv_np(const r4d_gemv_args& a, const GemvForm& f) {
   launch_gemv_a<KB, MT, 2, 4>(a);
 }
 
-// Here A's slice is staged whole: more than one row tile, or a slice past kAldsMax, runs here only with the fused transform,
-// and in trellis_mid.hip, which stages it in chunks, otherwise (16 rows, the slice past the limit, us when each wave read
-// its fragments from L2 instead -> now: 5120 x 34816 48.8 -> 41.7, 17408 x 5120 29.1 -> 26.6, KB 5 5120 x 16384 27.6 -> 22.1).
+// Here A's slice is staged whole; a slice past kAldsMax goes to trellis_mid.hip, which stages it in chunks (16 rows, us when
+// each wave read its fragments from L2 instead -> now: 5120 x 34816 48.8 -> 41.7, 17408 x 5120 29.1 -> 26.6, KB 5 5120 x 16384
+// 27.6 -> 22.1). Above 16 rows a slice that fits is faster here in the one-wave order -- no chunk barriers, one wait before the
+// first step (chunked / whole: 17 rows 1024 x 2048 11.9 / 10.6 us, 40 rows 512 x 2048 10.0 / 9.4, 64 rows 256 x 512 9.1 / 8.5;
+// 0.8 to 1.03 of the time over 128..1280 k, 1024..16384 columns and all rates). In the 4-wave order it is so to 32 rows where
+// a part has an odd number of steps, half of the last two-step chunk being waste there (24 rows 6144 x 5120 in 8 slices 18.2 /
+// 16.0; an even number 0.92 to 1.16), and not above (1.3 to 1.5 on full grids: two workgroups' worth of LDS and registers).
 template <int KB>
 void launch_gemv_kb(const r4d_gemv_args& a, const char* entry) {
   const GemvForm f = gemv_form(a.M, a.N, a.SKG, a.ws != 0 && a.tickets != 0, a.sk1 != 0, a.xf != 0);
-  const bool whole = f.MT == 1 && gemv_ktl_pad(f.SK, a.K / 16 / a.SKG) * a.M * 32 <= kAldsMax;
+  const size_t pad = gemv_ktl_pad(f.SK, a.K / 16 / a.SKG);
+  const bool whole = pad * a.M * 32 <= kAldsMax && (f.MT == 1 || f.SK == 1 || (f.MT == 2 && (pad / 16) % 2 == 1));
   if (!a.xf && !whole) r4d::gemv_mid(a, f.SK == 1, entry);
   else if (f.MT <= 1) launch_gemv_np<KB, 1>(a, f);
   else if (f.MT <= 2) launch_gemv_np<KB, 2>(a, f);

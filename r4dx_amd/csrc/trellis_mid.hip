@@ -1,6 +1,6 @@
-// trellis_mid.hip -- the trellis linear for 17..64 rows on gfx950 (r4d_gemm_trellis_nt_m64 and its _raw, _wq, _parts and
-// no-allocation forms above 16 rows): the batch, and the tail of a prompt. Also up to 16 rows where a K slice of A does not
-// fit the LDS whole (trellis_gemv.hip's rule).
+// trellis_mid.hip -- the trellis linear where a K slice of A does not fit the LDS whole, and for most of 17..64 rows, on gfx950
+// (r4d_gemm_trellis_nt_m64 and its _raw, _wq, _parts and no-allocation forms; trellis_gemv.hip has the rule): the batch, and the
+// tail of a prompt.
 //
 // DESIGN (MI355X): the decode (about 4 VALU lane-ops per weight) bounds this range, as it does for fewer rows; the MFMAs
 // (2 to 4 row tiles) take a quarter to a half of its time. So the decode stays the GEMV's -- each wave decodes one tile pair

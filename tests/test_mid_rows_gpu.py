@@ -1,6 +1,7 @@
-"""r4d_gemm_trellis_nt_m64 in the chunked kernel (trellis_mid.hip: 17..64 rows, and fewer where a K slice of A is past 48 KiB) at
-the sizes where its staging, its row tiles and its balanced form can go wrong. Each row must carry the bits the same launch
-gives it in a batch whose slice of A stays within 48 KiB -- the kernel that stages A whole, which shares neither the chunks nor
+"""r4d_gemm_trellis_nt_m64 above 16 rows, and below where a K slice of A is past 48 KiB: the chunked kernel (trellis_mid.hip)
+and the forms of two and more row tiles that stage the slice whole, at the sizes where their staging, their row tiles and
+the balanced form can go wrong. Each row must carry the bits the same launch
+gives it in a batch of at most 16 whose slice of A stays within 48 KiB -- one row tile, A staged whole: neither the chunks nor
 the cuts -- in both summation orders, at every rate, for slices whose last step is not whole, parts that are empty or shorter
 than the others, two input parts and more than 8 slices. The balanced form (cut units) at every number of row tiles and every
 rate, at one slice and at two; unsplit, it must also match the launch without ws and tickets, which cuts nothing, and stay
@@ -24,6 +25,9 @@ CASES = [   # (M, K, N, KB, SKG, sk)
     (49, 1152, 256, 3, 9, 2), (64, 2048, 384, 5, 16, 2), (64, 5120, 128, 4, 1, 1), (31, 4992, 256, 4, 3, 2),
     (18, 128, 128, 4, 1, 0), (32, 640, 256, 5, 5, 4), (48, 384, 128, 3, 3, 0), (49, 2304, 256, 5, 2, 0),
     (64, 4992, 256, 4, 1, 0), (57, 1152, 128, 4, 9, 0), (64, 128, 128, 5, 8, 0),
+    # slices whose last step is not whole, in the chunked kernel: past 48 KiB, and parts of an even number of steps
+    (64, 3456, 256, 5, 8, 2), (40, 5760, 128, 4, 8, 2), (23, 9856, 128, 3, 8, 1), (50, 1664, 256, 4, 8, 0), (20, 3456, 128, 4, 8, 0),
+    (32, 3456, 256, 5, 8, 4),
     # balanced (40 steps a unit): columns -n are column groups such that there are n SKG more units than CUs (rounded down)
     (29, 2560, -1, 4, 1, 2), (64, 2560, -44, 4, 1, 2), (37, 2560, -5, 3, 1, 2), (13, 2560, -3, 5, 1, 2), (10, 2560, -2, 4, 1, 1),
     (58, 2560, -2, 5, 1, 1), (37, 5120, -12, 5, 2, 2), (57, 5120, -3, 4, 2, 2), (20, 5120, -2, 3, 2, 1), (16, 5120, -5, 4, 2, 2),
