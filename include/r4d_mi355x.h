@@ -32,9 +32,9 @@ extern "C" {
  * ws fp32 ws_bytes(M, N, SKG) (SKG M N 4 at most 2 GiB), tickets tickets_bytes(N) (one 128-byte line per
  * 128-column group) zeroed before first use (self-resetting). One launch in flight per ws and tickets, whatever SKG: where
  * both are given, an unsplit launch (SKG = 1) uses them too -- the 4-wave order always; the SK 1 / 2 order, at any M, when
- * there are more column groups than compute units (not a multiple), K >= 2560, and A does not fit a workgroup whole (above 16
- * rows, or M K 2 bytes past 48 KiB): groups cut between workgroups are handed on through M N 4 bytes of ws and a word per
- * workgroup of the tickets. Without ws or tickets that order cuts nothing and gives the same bits. */
+ * there are more column groups than compute units (not a multiple), K >= 2560 and A takes more than 48 KiB (M K 2 bytes):
+ * groups cut between workgroups are handed on through M N 4 bytes of ws and a word per workgroup of the tickets. Without ws
+ * or tickets that order cuts nothing and gives the same bits. */
 void r4d_gemm_trellis_nt_m64(int64_t a0, int64_t a1, int n_split, int64_t w, int64_t svh, int64_t c,
                              int64_t ws, int64_t tickets, int M, int K, int N, int KB, int WV, int SK,
                              int MT, int NP, int SKG, int U, int NT, float out_scale, int64_t stream);
