@@ -52,8 +52,9 @@ __global__ __launch_bounds__(256) void tq_input_kernel(R4XSrc src, long long K, 
 }
 // E = 8 is the form with the fewest instructions per element; a launch too small to give every SIMD a wave of it (fewer
 // than 4096 items) is latency-bound and takes E = 2 in one-wave workgroups: a quarter of each lane's serial work, four
-// times the waves (one row of 17408 through silu: 4.0 us at best at E = 8, 2.6 at E = 2; 256 rows: 10.6 us at E = 8, 13.7 at two
-// elements per lane, all stages through the LDS crossbar).
+// times the waves. Against two elements 64 apart per lane with two stages through the LDS crossbar, in graphs of the one
+// launch: 1 x 17408 through silu 2.11 -> 1.88 us, 8 x 5120 with 3 outputs 2.06 -> 1.99, 29 x 17408 through silu 3.13 -> 2.80;
+// at E = 8 256 x 17408 through silu 13.7 -> 10.4.
 constexpr int64_t kWideItems = 4096;
 template <int SRC, bool BF16>
 void input_launch(const R4XSrc& src, int64_t rows, int64_t K, int nout, const OutPtrs& p, float scale, hipStream_t st) {
