@@ -128,8 +128,8 @@ constexpr size_t tq_end_lds(int MT, int NPW, int SK, int M) { return tq_end_lds_
 //   * else the partials go to ws -- above one row tile through LDS, as 16-byte row pieces (the accumulators' own 4-byte
 //     stores cost 3 to 5 us a launch at 49 and 64 rows) -- and the last of the group's SKG 4 / NPW contributors (ticket)
 //     sums the slices: run p (0..7) is 0.f + slices p, p + 8, ... in order, then the runs in order 0..7 (an absent slice
-//     adds +0.f, which changes nothing) -- the same arithmetic for every element whatever M is. The loads are coherent (sc1) 16-byte buffer loads,
-//     every slice of a batch of 8 requested before any is added.
+//     adds +0.f, which changes nothing) -- the same arithmetic for every element whatever M is. The loads are coherent
+//     (sc1) 16-byte buffer loads, every slice of a batch of 8 requested before any is added.
 // Each 32-lane half of a wave then owns one row's 128 sums, 4 adjacent columns per lane, from the slice sum to the
 // store (r4_fwht128_rows): no LDS copy of the slice sums, no stage through the LDS crossbar and one 8-byte store per lane.
 // STAGE: also one row tile above 8 rows goes through LDS.

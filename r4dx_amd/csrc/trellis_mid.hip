@@ -7,8 +7,8 @@
 // straight into MFMA B fragments, nothing of it passes through LDS -- and only A is shared: the workgroup stages it in
 // LDS, in MFMA operand order, a chunk of CS 64-k steps at a time in two buffers, so a row is read from L2 once per
 // workgroup and not once per wave. (Each wave reading its own A fragments from L2, which this replaces, waited for them:
-// MT x 2 KiB of scattered 32-byte pieces per 1 KiB of weights. Before -> now, 29 rows: 5120 x 34816 94 -> 52 us, 17408 x
-// 5120 52 -> 33; 64 rows: 171 -> 67 and 97 -> 45; 49 rows, KB 5: 5120 x 16384 60 -> 33, 6144 x 5120 52 -> 26. What is left
+// MT x 2 KiB of scattered 32-byte pieces per 1 KiB of weights. Before -> now, 29 rows: 5120 x 34816 95 -> 49 us, 17408 x
+// 5120 52 -> 33; 64 rows: 171 -> 68 and 97 -> 47; 49 rows, KB 5: 5120 x 16384 60 -> 34, 6144 x 5120 52 -> 26. What is left
 // over the decode's own time is one wave per SIMD's latencies (0.5 us a step at two row tiles, 0.25 of it decode issue) and
 // 9 to 15 us of launch, first loads and split hand-over.)
 //

@@ -421,8 +421,9 @@ __global__ __launch_bounds__(64 * kWaves, MR <= 8 ? (G == 32 ? 8 : 6) : 1) void 
         for (int u = 0; u < 4 / NG; ++u) {
           const int c = G == 64 ? (u & 1) * 2 + (u >> 1) : g + 2 * u, ch = u & (kCh - 1);
           const Acc t0 = u < kCh ? Acc{} : t[ch];
-          if constexpr (SMALL) t[ch] = __builtin_amdgcn_mfma_f32_16x16x32_f16(afrag(i, kbl, c), w4_bop(bq, c), t0, 0, 0, 0);
-          else t[ch] = __builtin_amdgcn_mfma_f32_32x32x16_f16(u < kEarlyA ? af[u < kEarlyA ? u : 0] : afrag(i, kbl, c), w4_bop(bq, c), t0, 0, 0, 0);
+          const r4h8 fa = u < kEarlyA ? af[u < kEarlyA ? u : 0] : afrag(i, kbl, c);
+          if constexpr (SMALL) t[ch] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa, w4_bop(bq, c), t0, 0, 0, 0);
+          else t[ch] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa, w4_bop(bq, c), t0, 0, 0, 0);
         }
         if constexpr (SMALL) {
           // output rows 4 (lane >> 4) + e = 2 m + t: tile t = e & 1 (rows m >= M have zero A and stay 0)
